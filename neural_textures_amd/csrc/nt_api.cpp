@@ -1592,6 +1592,65 @@ static int fwd_common(const nt_latents *lat, const nt_mlp *mlp, bool need_latent
     return NT_OK;
 }
 
+// The strip kernel's descriptor (nt_infer.hip) for a validated inference call; false where
+// only the general kernel applies: textures that are not one to four of the image's size
+// with float4 texels, images of less than four texels a side (taps wrap at most once) or
+// more than 2^20 (a texel centre's fp32 position is then no longer within half a texel), and
+// grids or images past 32-bit offsets.
+static bool infer_desc(const nt_params *p, const FwdDesc &f, InferDesc &d)
+{
+    const int W = p->image_width, H = p->image_height, C = f.C;
+    if (W < 4 || H < 4 || W > (1 << 20) || H > (1 << 20) || p->num_textures < 1 || p->num_textures > 4)
+        return false;
+    d = InferDesc{};
+    d.mlp = f.mlp;
+    d.G = f.G;
+    for (int gi = 0; gi < NT_MAX_GRIDS; ++gi) {
+        const GridDesc &g = f.grid[gi < f.G ? gi : 0];
+        if ((int64_t)g.w * g.h * C >= (1ll << 31))
+            return false;
+        d.grid[gi].values = g.values + g.mip_off[0] * C;
+        d.grid[gi].w = g.w;
+        d.grid[gi].h = g.h;
+    }
+    int out = 0;
+    for (int t = 0; t < 4; ++t) {
+        const TexDesc &x = f.tex[t < p->num_textures ? t : 0];
+        if (!x.texels || x.pitch != 4 || x.w != W || x.h != H)
+            return false;
+        d.tex[t] = x.texels;
+        d.tex_nch[t] = t < p->num_textures ? x.nch : 0;
+        d.tex_out0[t] = t < p->num_textures ? out : 0;
+        out += d.tex_nch[t];
+    }
+    d.ntex = p->num_textures;
+    d.image_w = W;
+    d.image_h = H;
+    d.inv_w = f.inv_w;
+    d.inv_h = f.inv_h;
+    d.out32 = f.out32;
+    d.out_stride = f.out_stride;
+    d.inv_stride = 1.f / (float)f.out_stride;
+    d.sse = f.sse;
+    // A strip reads four texture rows more than it has. Sixteen rows where that leaves every
+    // SIMD's two waves four strips each (2048^2: 178 us, 192 us with eight; 2047 x 1111, which
+    // would leave two: 262 us, 250 with eight), else eight, and fewer while the strips do not
+    // give every SIMD four.
+    d.strips_x = (W + 31) / 32;
+    auto strips_of = [&](int rows) { return (int64_t)d.strips_x * ((H + rows - 1) / rows); };
+    const int64_t waves = 4 * (int64_t)device_cu_count(); // one per SIMD
+    d.rows = strips_of(16) >= 8 * waves ? 16 : 8;
+    while (d.rows > 1 && strips_of(d.rows) < 4 * waves)
+        d.rows /= 2;
+    d.strips_y = (H + d.rows - 1) / d.rows;
+    // At most one partial sum a workgroup: never more than the caller's workspace holds
+    // (nt_inference_workspace_bytes).
+    const int64_t strips = (int64_t)d.strips_x * d.strips_y;
+    d.blocks = (int)std::min<int64_t>((strips + kFwdWaves - 1) / kFwdWaves,
+                                      std::min(kFwdMaxBlocks, forward_blocks(f.count) * kFwdWaves));
+    return true;
+}
+
 int nt_inference(const nt_params *p, void *stream)
 {
     if (!p)
@@ -1620,19 +1679,25 @@ int nt_inference(const nt_params *p, void *stream)
     d.out32 = p->inference_output;
     d.sse = p->inference_mse_accum;
     d.out_stride = p->mlp.sizes[p->mlp.num_layers];
-    const int partials = forward_blocks(d.count) * kFwdWaves;
-    if (p->workspace && p->workspace_bytes >= (size_t)partials * sizeof(float)) {
+    const size_t ws_need = (size_t)forward_blocks(d.count) * kFwdWaves * sizeof(float);
+    float *sse_partial = nullptr;
+    if (p->workspace && p->workspace_bytes >= ws_need) {
         if (!aligned16(p->workspace))
             return fail(NT_ERR_MISALIGNED, "workspace must be 16-byte aligned");
-        d.sse_partial = (float *)p->workspace;
+        sse_partial = (float *)p->workspace;
     }
+    InferDesc q;
+    const bool strips = infer_desc(p, d, q);
+    d.sse_partial = q.sse_partial = sse_partial;
     hipError_t e;
     {
         ProfileScope prof((hipStream_t)stream);
-        e = launch_forward(shape, kFwdInference, d, (hipStream_t)stream);
+        e = strips ? launch_inference(shape, q, (hipStream_t)stream)
+                   : launch_forward(shape, kFwdInference, d, (hipStream_t)stream);
     }
-    if (e == hipSuccess && d.sse_partial)
-        e = launch_sse_reduce(d.sse_partial, partials, d.sse, (hipStream_t)stream);
+    if (e == hipSuccess && sse_partial)
+        e = launch_sse_reduce(sse_partial, strips ? q.blocks : forward_blocks(d.count) * kFwdWaves, d.sse,
+                              (hipStream_t)stream);
     return hip_status(e, "inference launch");
 }
 

@@ -466,32 +466,6 @@ __global__ __launch_bounds__(kFwdThreads, fwd_min_blocks<MODE>()) void forward_k
     }
 }
 
-// The fixed-order SSE reduction: thread t sums partial[t], partial[t + 256], ... in index
-// order, then a pairwise tree over the 256 sums; the result is the same bits on every run.
-__global__ __launch_bounds__(256) void sse_reduce_kernel(const float *partial, int n, float *sse)
-{
-    __shared__ float part[256];
-    const int t = threadIdx.x;
-    float s = 0.f;
-    for (int i = t; i < n; i += 256)
-        s += partial[i];
-    part[t] = s;
-    __syncthreads();
-    for (int w = 128; w > 0; w >>= 1) {
-        if (t < w)
-            part[t] += part[t + w];
-        __syncthreads();
-    }
-    if (t == 0)
-        sse[0] = sse[0] + part[0];
-}
-
-hipError_t launch_sse_reduce(const float *partial, int n, float *sse, hipStream_t s)
-{
-    hipLaunchKernelGGL(sse_reduce_kernel, dim3(1), dim3(256), 0, s, partial, n, sse);
-    return hipGetLastError();
-}
-
 // ---- LDS-staged decode (second pass of the two-pass decode) ----------------------------
 // Same per-pixel arithmetic as forward_kernel<..., Decode16> (and so the same bits): the
 // corner texels come from per-block LDS boxes instead of HBM/L2. Box entry of (grid, mip):

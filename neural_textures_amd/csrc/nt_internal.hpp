@@ -358,6 +358,30 @@ struct FwdDesc {
     float jitter, mip_min, mip_max;
 };
 
+// Full-image inference with reference textures of the image's size (nt_infer.hip): strips of
+// 32 pixels x `rows` rows, one wave each.
+struct InferGrid {
+    const float *values; // mip 0, [texel][C]
+    int w, h;
+};
+struct InferDesc {
+    MlpDesc mlp;
+    InferGrid grid[NT_MAX_GRIDS]; // entries past G repeat grid 0
+    int G;
+    const float *tex[4]; // float4 texels, image size; entries past ntex repeat texture 0
+    int tex_nch[4];      // 0 past ntex
+    int tex_out0[4];     // output of the texture's first channel
+    int ntex;
+    int image_w, image_h;
+    float inv_w, inv_h; // 1/image_w, 1/image_h when powers of two (exact), else 0 (divide)
+    int rows, strips_x, strips_y, blocks;
+    float *out32;
+    int out_stride;
+    float inv_stride;
+    float *sse;
+    float *sse_partial; // one per workgroup (NULL: atomics)
+};
+
 struct AdamDesc {
     float beta1, beta2, lr, eps, bc1, bc2;
 };
@@ -444,6 +468,7 @@ __host__ __device__ inline int box_last(int b1, int image, float jitter, int lev
 }
 hipError_t launch_decode_box(int shape, const DecodeBoxDesc &d, hipStream_t s);
 size_t decode_box_weight_bytes(int shape);
+hipError_t launch_inference(int shape, const InferDesc &d, hipStream_t s);
 // *sse += the sum of partial[0..n) in a fixed order (one workgroup).
 hipError_t launch_sse_reduce(const float *partial, int n, float *sse, hipStream_t s);
 hipError_t launch_net_adam(const NetAdamDesc &d, hipStream_t s);

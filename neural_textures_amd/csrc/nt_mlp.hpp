@@ -141,6 +141,101 @@ __device__ h8 weight_fragment(const MlpDesc &m, int idx)
     return v;
 }
 
+// Layer-0 input feature of element e of k-step fragment q in lane group g for networks on
+// C-channel grids. 16 channels: grid_feature (grids g and g + 2, eight consecutive channels
+// per fragment). 3 channels (up to four grids, one k-step): lane group g holds grid g's
+// channels (e = 0..2), grid g + 2's (e = 3..5) and two of the padding features 12..15
+// (e = 6, 7), so that each lane samples two grids and the two groups together cover all
+// sixteen inputs. 8 channels (up to two grids): grid g's channels, the natural order.
+template <int C>
+__host__ __device__ constexpr int input_feature(int q, int g, int e)
+{
+    if constexpr (C == 16)
+        return grid_feature(q, g, e);
+    else if constexpr (C == 3)
+        return e < 3 ? 3 * g + e : e < 6 ? 3 * (g + 2) + (e - 3) : 12 + 2 * g + (e - 6);
+    else
+        return 16 * q + 8 * g + e;
+}
+
+// Layer l's forward fragments, items tid, tid + NT, ... (an item is a fragment's lane): a
+// lane's eight inputs of one output row are 16 consecutive bytes of the weight row (layer 0;
+// with 3 channels eight scattered halves) or two runs of 8 bytes (chained order), so the
+// fragments are read with those loads, all of them issued before the first LDS store.
+template <class S, int C, int l, int NT>
+__device__ __forceinline__ void stage_forward_layer(const MlpDesc &m, h8 *frags, int tid)
+{
+    constexpr int kin = S::kin(l), kout = S::kout(l), qn = kin / 16;
+    constexpr int items = S::fwd_frags(l) * kWave, N = (items + NT - 1) / NT;
+    const uint16_t *W = m.W[l];
+    h8 v[N];
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+        const int idx = min(tid + j * NT, items - 1), f = idx / kWave, lane = idx % kWave;
+        const int c = lane & 31, g = lane >> 5, a = f / qn, q = f % qn;
+        const int n = 32 * a + c;
+        const uint16_t *row = W + min(n, kout - 1) * kin;
+        if constexpr (l > 0) {
+            const uint2 lo = load_global((const uint2 *)(row + chained_feature(q, g, 0)));
+            const uint2 hi = load_global((const uint2 *)(row + chained_feature(q, g, 4)));
+            v[j] = __builtin_bit_cast(h8, make_uint4(lo.x, lo.y, hi.x, hi.y));
+        } else if constexpr (C == 3) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e)
+                v[j][e] = bits_h(load_global(row + input_feature<C>(q, g, e)));
+        } else {
+            v[j] = __builtin_bit_cast(h8, load_global((const uint4 *)(row + input_feature<C>(q, g, 0))));
+        }
+        if (n >= kout)
+            v[j] = (h8)(_Float16)0.f;
+    }
+#pragma unroll
+    for (int j = 0; j < N; ++j)
+        if (tid + j * NT < items)
+            frags[S::fwd_off(l) * kWave + tid + j * NT] = v[j];
+}
+
+// Stage the forward weight fragments and fp32 biases of a network on C-channel grids
+// (input_feature order) in LDS, NT threads; the caller synchronises afterwards. Weights that
+// are not 16-byte aligned are read element by element.
+template <class S, int C, int NT>
+__device__ __forceinline__ void stage_forward(const MlpDesc &m, h8 *frags, float *bias, int tid)
+{
+    uintptr_t mis = 0;
+#pragma unroll
+    for (int l = 0; l < S::L; ++l)
+        mis |= (uintptr_t)m.W[l] & 15u;
+    if (mis == 0) {
+        stage_forward_layer<S, C, 0, NT>(m, frags, tid);
+        stage_forward_layer<S, C, 1, NT>(m, frags, tid);
+        if constexpr (S::L > 2)
+            stage_forward_layer<S, C, 2, NT>(m, frags, tid);
+        if constexpr (S::L > 3)
+            stage_forward_layer<S, C, 3, NT>(m, frags, tid);
+        static_assert(S::L <= 4, "at most four layers");
+    } else {
+        for (int idx = tid; idx < S::fwd_total() * kWave; idx += NT) {
+            const int f = idx / kWave, lane = idx % kWave, c = lane & 31, g = lane >> 5;
+            int l = 0;
+            while (l + 1 < S::L && f >= S::fwd_off(l + 1))
+                ++l;
+            const int kin = S::kin(l), qn = kin / 16, local = f - S::fwd_off(l);
+            const int n = 32 * (local / qn) + c, q = local % qn;
+            h8 v;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const int k = l > 0 ? chained_feature(q, g, e) : input_feature<C>(q, g, e);
+                v[e] = n < S::kout(l) ? bits_h(m.W[l][n * kin + k]) : (_Float16)0.f;
+            }
+            frags[idx] = v;
+        }
+    }
+#pragma unroll
+    for (int l = 0; l < S::L; ++l)
+        for (int n = tid; n < 32 * S::t32(S::kout(l)); n += NT)
+            bias[S::bias_off(l) + n] = n < m.sizes[l + 1] ? h2f(m.B[l][n]) : 0.f;
+}
+
 // fp32 bias row idx (layers back to back, each padded to 32-row tiles).
 template <class S>
 __device__ float bias_value(const MlpDesc &m, int idx)

@@ -93,20 +93,6 @@ __host__ __device__ constexpr int raw_off(int l)
     return o;
 }
 
-// Layer-0 input feature of element e of k-step fragment q in lane group g. 16 channels:
-// grid_feature (grids g and g + 2, eight consecutive channels per fragment). 3 channels
-// (four grids, one k-step): lane group g holds grid g's channels (e = 0..2), grid g + 2's
-// (e = 3..5) and two of the padding features 12..15 (e = 6, 7), so that each lane samples
-// two grids and the two groups together cover all sixteen inputs.
-template <int C>
-__host__ __device__ constexpr int input_feature(int q, int g, int e)
-{
-    if constexpr (C == 16)
-        return grid_feature(q, g, e);
-    else
-        return e < 3 ? 3 * g + e : e < 6 ? 3 * (g + 2) + (e - 3) : 12 + 2 * g + (e - 6);
-}
-
 // Output index of output row r (r < 16): nibble r of the packed permutation.
 __device__ __forceinline__ int perm_row(uint64_t perm, int r) { return (int)((perm >> (4 * r)) & 15u); }
 

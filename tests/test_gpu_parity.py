@@ -467,6 +467,54 @@ def test_inference(lib, O, shape):
         1e-2 * abs(float(st.inference_mse_accum[0]))
 
 
+# (network, image size, textures' channels, texture size as the image's or another): strips of
+# one pixel and of 32, 33 and 31 (whole, one over, one short), row counts around the five-row
+# window, the smallest image the strip kernel takes (4 x 4) and one below it, sizes whose texel
+# centres are not exact in fp32, output rows of 16, 9, 12 and 3 floats, one to five textures.
+INFERENCE_CASES = [
+    ("ref", (4, 4), [3, 3, 3], False), ("ref", (3, 9), [3, 3, 3], False), ("ref", (32, 16), [3, 3, 3], False),
+    ("ref", (33, 7), [4, 4], False), ("ref", (31, 40), [1], False), ("ref", (100, 61), [3, 4, 2, 4], False),
+    ("ref", (40, 24), [3, 3, 3], True), ("ref", (40, 24), [3, 3, 1, 1, 1], False),
+    ("c1", (37, 21), [3], False), ("c2", (95, 50), [3, 3, 3], False), ("c2", (4, 129), [4, 2], False),
+    ("c4", (65, 33), [4, 4, 4], False), ("c4", (129, 5), [3], False),
+]
+
+
+@pytest.mark.parametrize("shape,size,tex,other_size", INFERENCE_CASES)
+def test_inference_strips(lib, O, shape, size, tex, other_size):
+    """Outputs as the oracle's, with and without a workspace; the SSE within 4e-3 (an output
+    differs by at most an fp16 rounding, 2^-11 of its value, which changes its squared error by
+    2 |y| / |y - t| times that, and the errors here are of the outputs' size)."""
+    import torch
+    say(f"case: inference strips {shape} {size} textures {tex} other size {other_size}")
+    w, h = size
+    rng = np.random.default_rng(w * 1000 + h)
+    st = make_state(shape, image=64, region=(16, 16), seed=w)
+    for l in range(st.net.num_layers):
+        st.net.biases[l] = P.f16_bits(rng.uniform(-0.1, 0.1, st.net.sizes[l + 1]))
+    st.image_width, st.image_height = w, h
+    tw, th = (2 * w, h) if other_size else (w, h)
+    st.textures = [P.make_texture(tw, th, c, rng.uniform(0, 1, (th, tw, 4)).astype(np.float32)) for c in tex]
+    for t in st.textures:  # float4 texels for one channel too (five textures keep pitch 1)
+        if t.pitch == 1 and len(tex) < 5:
+            t.texels, t.pitch = np.repeat(t.texels, 4), 4
+    no = st.net.sizes[-1]
+    st.inference_output = np.zeros(w * h * no, np.float32)
+    st.inference_mse_accum = np.zeros(1, np.float32)
+    gs = st.to_torch()
+    assert O.ntref_inference(C.byref(st.params())) == 0
+    want = float(st.inference_mse_accum[0])
+    for ws in (False, True):
+        need = lib.nt_inference_workspace_bytes(C.byref(gs.params()))
+        gs.workspace = torch.empty(need, dtype=torch.uint8, device="cuda") if ws else None
+        gs.inference_output.fill_(float("nan"))
+        gs.inference_mse_accum.zero_()
+        nt.check(lib.nt_inference(C.byref(gs.params()), None))
+        sync()
+        assert_close(gs.inference_output, st.inference_output, "inference output")
+        assert abs(float(to_np(gs.inference_mse_accum)[0]) - want) <= 4e-3 * want
+
+
 def test_inference_sse_fixed_order(lib, O):
     """With a workspace the SSE is summed in a fixed order: the same bits on every run, and
     within rounding of the atomic path and of the oracle's float64 sum."""
