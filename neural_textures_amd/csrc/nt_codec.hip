@@ -4,9 +4,9 @@
 //
 // Encode: one thread per (block, channel). Endpoints are the min and max order key of the
 // block's fp16-rounded values; each index minimises |v - decode(i)| in fp32 (lowest index
-// wins ties), found by binary searches over the 16 decoded levels. Integer key arithmetic
-// plus IEEE fp32 compares make the result bit-exact against the CPU restatement (a linear
-// scan). Decode: one thread per (texel, 4 channels), float4 stores.
+// wins ties), found among three candidate levels, or by binary searches over the 16 decoded
+// levels where levels can coincide. Integer key arithmetic plus IEEE fp32 compares make the
+// result bit-exact against the CPU restatement (a linear scan). Decode: one thread per (texel, 4 channels), float4 stores.
 #include <algorithm>
 
 #include "nt_internal.hpp"
@@ -23,11 +23,15 @@ namespace ntk {
 // finds the first. N searches run step by step together, so each step's N LDS reads are
 // issued at once.
 //
-// R is the thread's padded level row: R[0] = R[1] = L[0], R[2 + i] = L[i], R[18] = L[15],
-// so levels j - 2, j - 1 and j (clamped to the ends) are R[j], R[j + 1], R[j + 2] for every
-// j in [0, 16] without index clamps; at j = 0 and j = 16 levels j - 1 and j read equal, so
-// the comparison between them picks j - 1 (clamped to 0) as it must.
-constexpr int kLevelRow = 19; // padded row length; odd, so threads' rows fall in distinct banks
+// R is the thread's padded level column: R[0] = R[1] = L[0], R[2 + i] = L[i], R[18] = L[15]
+// (entries kLevelStride floats apart), so levels j - 2, j - 1 and j (clamped to the ends) are
+// R[j], R[j + 1], R[j + 2] for every j in [0, 16] without index clamps; at j = 0 and j = 16
+// levels j - 1 and j read equal, so the comparison between them picks j - 1 (clamped to 0) as
+// it must. A thread's entries are one workgroup (256 floats) apart, so they all lie in the
+// thread's own LDS bank: reads at any level are free of conflicts (with a row per thread, the
+// levels side by side, the lanes' reads fell in random banks).
+constexpr int kLevelRows = 19;
+constexpr int kLevelStride = 256;
 
 typedef unsigned short us2 __attribute__((ext_vector_type(2)));
 typedef short s2 __attribute__((ext_vector_type(2)));
@@ -38,22 +42,22 @@ __device__ __forceinline__ void codec_nearest_n(const float *R, const float *v, 
     const float *q[N];
 #pragma unroll
     for (int p = 0; p < N; ++p)
-        q[p] = R + 2;
+        q[p] = R + 2 * kLevelStride;
 #pragma unroll
     for (int step = 8; step > 0; step >>= 1) {
         float l[N];
 #pragma unroll
         for (int p = 0; p < N; ++p)
-            l[p] = q[p][step - 1];
+            l[p] = q[p][(step - 1) * kLevelStride];
 #pragma unroll
         for (int p = 0; p < N; ++p)
-            q[p] += l[p] < v[p] ? step : 0;
+            q[p] += l[p] < v[p] ? step * kLevelStride : 0;
     }
     float lm[N], lc[N], l2[N];
 #pragma unroll
     for (int p = 0; p < N; ++p) {
-        l2[p] = q[p][-2];
-        lm[p] = q[p][-1];
+        l2[p] = q[p][-2 * kLevelStride];
+        lm[p] = q[p][-kLevelStride];
         lc[p] = q[p][0];
     }
     float a[N];
@@ -61,7 +65,7 @@ __device__ __forceinline__ void codec_nearest_n(const float *R, const float *v, 
     bool need[N], any = false;
 #pragma unroll
     for (int p = 0; p < N; ++p) {
-        j[p] = (int)(q[p] - (R + 2));
+        j[p] = (int)(q[p] - (R + 2 * kLevelStride)) / kLevelStride;
         a[p] = fabsf(v[p] - lm[p]);
         const bool upper = fabsf(v[p] - lc[p]) < a[p];
         idx[p] = upper ? j[p] : max(j[p] - 1, 0);
@@ -78,7 +82,7 @@ __device__ __forceinline__ void codec_nearest_n(const float *R, const float *v, 
 #pragma unroll
         for (int it = 0; it < 4; ++it) {
             const int mid = (lo + hi) >> 1;
-            const bool le = fabsf(v[p] - R[2 + mid]) <= a[p];
+            const bool le = fabsf(v[p] - R[(2 + mid) * kLevelStride]) <= a[p];
             hi = lo < hi && le ? mid : hi;
             lo = lo < hi && !le ? mid + 1 : lo;
         }
@@ -86,53 +90,92 @@ __device__ __forceinline__ void codec_nearest_n(const float *R, const float *v, 
     }
 }
 
+// The same indices where the order keys k0 .. k1 of a block's values span at least
+// kCandidateSpan: three candidate levels per value instead of a search. Level m's key is
+// k0 + round(kd w_m / 64), kd = k1 - k0, w_m = round(64 m / 15), so in steps of kd / 15 it
+// lies within D = 7/64 + 7.5/kd of m (0.344 at kd = 32). For a value whose fp16 key lies
+// p steps above k0, levels m < p - D are below it and levels m > p + D are not, so with
+// i = floor(p - D') (D' = 0.36: D and the fp32 arithmetic's error, below 0.004) the levels
+// j - 1 and j around it (j levels below the value) are among i, i + 1, i + 2: i <= j - 1, and
+// i + 2 >= j as D + D' < 1. Neighbouring levels are at least one key apart, and at most 2^10
+// times as far apart in value as the next pair, so no two errors on one side of the value
+// are equal after fp32 rounding, and counting the strict improvements along the three gives
+// the first index of the least error. A value past the last level reads the row's padding
+// (level 15 again), which never improves.
+// What bounds the search: VALU issue (11 instructions a value against 26 for the binary
+// search) and the LDS reads (12 bytes a value against 28). 4096^2 x 16 channels of N(0, 0.5):
+// 310 -> 215 us, 5.9 TB/s of the 1.28 GB moved (VALU issue 80 % of the time, 398 instructions
+// a wave against 673); blocks of a smooth image, whose values span fewer keys and take the
+// binary search, 495 -> 490 us.
+constexpr uint32_t kCandidateSpan = 32;
+
+__device__ __forceinline__ int codec_nearest_candidate(const float *R, float v, float key, float scale, float bias)
+{
+    // scale = 15 / kd, bias = -(scale k0 + D'): below zero converts to 0.
+    // (a plain v_cvt_u32_f32, which clamps, without a float maximum before it).
+    uint32_t i;
+    asm("v_cvt_u32_f32 %0, %1" : "=v"(i) : "v"(fmaf(key, scale, bias)));
+    const float *q = R + (2 + i) * kLevelStride;
+    const float e0 = fabsf(v - q[0]), e1 = fabsf(v - q[kLevelStride]), e2 = fabsf(v - q[2 * kLevelStride]);
+    return (int)i + (e1 < e0) + (e2 < e1);
+}
+
 // Encode: a workgroup takes 256/C horizontally adjacent blocks of one block row, thread
 // (block, channel). The 16 decoded levels of a thread's (block, channel) are computed once
-// into its LDS row; each pixel's index is then a binary search over them. The nibbles are
+// into its LDS column; each pixel's index is then found among them (above). The nibbles are
 // assembled in LDS and stored as whole 32-bit words.
 template <int C>
 __global__ __launch_bounds__(256) void codec_encode_kernel(const float *values, int W, int H,
                                                            uint8_t *blocks)
 {
     constexpr int BPW = 256 / C; // blocks per workgroup
-    __shared__ float lev[256 * kLevelRow];
-    __shared__ uint8_t nib[BPW][16 * C];
+    __shared__ float lev[kLevelRows * kLevelStride];
+    __shared__ __align__(16) uint8_t nib[BPW][16 * C + 16]; // 16 bytes past a multiple of 256: other banks for each block
     const int tid = threadIdx.x, lb = tid / C, c = tid % C;
     const int bw = (W + 3) >> 2, bh = (H + 3) >> 2;
     const int bx = blockIdx.x * BPW + lb;
-    float *R = lev + tid * kLevelRow;
+    float *R = lev + tid;
+    const bool active = lb < BPW && bx < bw; // C = 12 leaves 256 % 12 threads idle
+    // A block's sixteen loads, from clamped (always valid) addresses, so that none sits under a
+    // branch waiting for its own round trip; pixels past the image edge are masked afterwards.
+    // Each row's base (the workgroup's first column) is uniform and the thread's byte offset
+    // in it is below 2^15: no address arithmetic per load.
+    const int x0 = 4 * BPW * (int)blockIdx.x;
+    uint32_t off[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+        off[q] = (uint32_t)(min(4 * lb + q, W - 1 - x0) * C + c) * 4u;
     for (int by = blockIdx.y; by < bh; by += gridDim.y) {
-        const bool active = lb < BPW && bx < bw; // C = 12 leaves 256 % 12 threads idle
         uint8_t *rec = blocks + ((int64_t)by * bw + bx) * (12 * C);
         if (active) {
-            // All sixteen loads first, from clamped (always valid) addresses, so that none
-            // sits under a branch waiting for its own round trip; pixels past the image
-            // edge are masked afterwards. Row bases are uniform, offsets 32-bit (W C < 2^31).
             float raw[16];
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                const float *row = values + (int64_t)min(4 * by + r, H - 1) * W * C;
+                const char *row = (const char *)(values + ((int64_t)min(4 * by + r, H - 1) * W + x0) * C);
 #pragma unroll
                 for (int q = 0; q < 4; ++q)
-                    raw[4 * r + q] = load_global(row + (min(4 * bx + q, W - 1) * C + c));
+                    raw[4 * r + q] = load_global((const float *)(row + off[q]));
             }
+            const bool whole = 4 * bx + 3 < W && 4 * by + 3 < H;
             float v[16];
+            us2 key[8]; // order keys, two pixels each
             uint32_t kmin = 0xFFFFu, kmax = 0u;
-            if (4 * bx + 3 < W && 4 * by + 3 < H) {
+            if (whole) {
                 // A block wholly inside the image (all but the last block row and column):
                 // the order keys two pixels per instruction (codec_key on each 16-bit half:
                 // h ^ 0xFFFF for a set sign bit, h ^ 0x8000 else), with packed min and max.
                 us2 kmn = {0xFFFF, 0xFFFF}, kmx = {0, 0};
 #pragma unroll
                 for (int p = 0; p < 16; p += 2) {
-                    v[p] = fminf(fmaxf(raw[p], -65504.f), 65504.f);
-                    v[p + 1] = fminf(fmaxf(raw[p + 1], -65504.f), 65504.f);
+                    // (a NaN gives the lower bound, as fmin(fmax()) does)
+                    v[p] = __builtin_amdgcn_fmed3f(raw[p], -65504.f, 65504.f);
+                    v[p + 1] = __builtin_amdgcn_fmed3f(raw[p + 1], -65504.f, 65504.f);
                     const f2 pv = {v[p], v[p + 1]};
                     const us2 hb = __builtin_bit_cast(us2, __builtin_convertvector(pv, h2));
                     const us2 sg = __builtin_bit_cast(us2, __builtin_bit_cast(s2, hb) >> (short)15);
-                    const us2 key = hb ^ ((sg & (unsigned short)0x7FFF) | (unsigned short)0x8000);
-                    kmn = __builtin_elementwise_min(kmn, key);
-                    kmx = __builtin_elementwise_max(kmx, key);
+                    key[p / 2] = hb ^ ((sg & (unsigned short)0x7FFF) | (unsigned short)0x8000);
+                    kmn = __builtin_elementwise_min(kmn, key[p / 2]);
+                    kmx = __builtin_elementwise_max(kmx, key[p / 2]);
                 }
                 kmin = kmn.x < kmn.y ? kmn.x : kmn.y;
                 kmax = kmx.x > kmx.y ? kmx.x : kmx.y;
@@ -144,20 +187,27 @@ __global__ __launch_bounds__(256) void codec_encode_kernel(const float *values, 
                     const uint32_t k = codec_key(h_bits((_Float16)v[p]));
                     kmin = in && k < kmin ? k : kmin;
                     kmax = in && k > kmax ? k : kmax;
+                    key[p >> 1][p & 1] = (unsigned short)k;
                 }
+                // Pixels past the edge: a key in range (their indices are written as 0).
+#pragma unroll
+                for (int p = 0; p < 16; ++p)
+                    if (!(4 * bx + (p & 3) < W && 4 * by + (p >> 2) < H))
+                        key[p >> 1][p & 1] = (unsigned short)kmin;
             }
             *(uint32_t *)(rec + 4 * c) = kmin | (kmax << 16);
             // The sixteen levels, two per instruction after the interpolation: key
-            // (64 k0 + (k1 - k0) w + 32) >> 6 (= codec_interp), then codec_unkey on each half
+            // (64 k0 + (k1 - k0) w + 32) >> 6 (= codec_interp), formed in the high half of
+            // (k0 << 16) + ((k1 - k0) w + 32) << 10, then codec_unkey on each half
             // (k ^ 0x8000 for a set top bit, k ^ 0xFFFF else) and the fp16 -> fp32 widening.
             float lv[16];
-            const uint32_t kbase = 64u * kmin + 32u, kd = kmax - kmin;
+            const uint32_t kbase = (kmin << 16) + (32u << 10), kd = kmax - kmin;
 #pragma unroll
             for (int i = 0; i < 16; i += 2) {
-                // kbase + kd w < 2^23: 24-bit products.
-                const uint32_t k0 = (kbase + __umul24(kd, (uint32_t)codec_weight(i))) >> 6;
-                const uint32_t k1 = (kbase + __umul24(kd, (uint32_t)codec_weight(i + 1))) >> 6;
-                const uint32_t kk = k0 | (k1 << 16);
+                // 24-bit factors: kd < 2^16, w << 10 <= 2^16.
+                const uint32_t k0 = kbase + __umul24(kd, (uint32_t)codec_weight(i) << 10);
+                const uint32_t k1 = kbase + __umul24(kd, (uint32_t)codec_weight(i + 1) << 10);
+                const uint32_t kk = __builtin_amdgcn_perm(k1, k0, 0x07060302u); // the high halves
                 // 0xFFFF in each half whose top bit is set (op_sel_hi: the shift count of the
                 // high half is the inline constant's low half too).
                 uint32_t top;
@@ -168,28 +218,44 @@ __global__ __launch_bounds__(256) void codec_encode_kernel(const float *values, 
                 lv[i + 1] = fv[1];
             }
             R[0] = lv[0];
-            R[1] = lv[0];
+            R[kLevelStride] = lv[0];
 #pragma unroll
             for (int i = 0; i < 16; ++i)
-                R[2 + i] = lv[i];
-            R[18] = lv[15];
+                R[(2 + i) * kLevelStride] = lv[i];
+            R[18 * kLevelStride] = lv[15];
             int idx[16];
-            codec_nearest_n<8>(R, v, idx);
-            codec_nearest_n<8>(R, v + 8, idx + 8);
+            // One of the two for the whole wave, so that a wave never runs both.
+            if (__ballot(kd < kCandidateSpan) == 0) {
+                const float scale = 15.f / (float)kd, bias = fmaf(-scale, (float)kmin, -0.36f);
 #pragma unroll
-            for (int p = 0; p < 16; ++p) {
-                const bool in = 4 * bx + (p & 3) < W && 4 * by + (p >> 2) < H;
-                nib[lb][p * C + c] = (uint8_t)(in ? idx[p] : 0);
+                for (int p = 0; p < 16; ++p)
+                    idx[p] = codec_nearest_candidate(R, v[p], (float)key[p >> 1][p & 1], scale, bias);
+            } else {
+                // Four searches at a time: 94 registers and five waves per SIMD (eight at a time:
+                // 110 and four, which costs both paths 8 %).
+#pragma unroll
+                for (int p = 0; p < 16; p += 4)
+                    codec_nearest_n<4>(R, v + p, idx + p);
             }
+            if (!whole) {
+#pragma unroll
+                for (int p = 0; p < 16; ++p)
+                    if (!(4 * bx + (p & 3) < W && 4 * by + (p >> 2) < H))
+                        idx[p] = 0;
+            }
+#pragma unroll
+            for (int p = 0; p < 16; ++p)
+                nib[lb][p * C + c] = (uint8_t)idx[p];
         }
         __syncthreads();
         if (active) {
             // Index area: nibble p*C + c; word w packs nibbles 8w .. 8w+7, low nibble first.
-            for (int w = c; w < 2 * C; w += C) {
-                uint32_t word = 0;
+            // x | x >> 4 puts each odd byte's nibble above the even byte's before it.
 #pragma unroll
-                for (int t = 0; t < 8; ++t)
-                    word |= (uint32_t)nib[lb][8 * w + t] << (4 * t);
+            for (int k = 0; k < 2; ++k) {
+                const int w = c + k * C;
+                const uint2 n = *(const uint2 *)&nib[lb][8 * w];
+                const uint32_t word = __builtin_amdgcn_perm(n.y | n.y >> 4, n.x | n.x >> 4, 0x06040200u);
                 *(uint32_t *)(rec + 4 * C + 4 * w) = word;
             }
         }

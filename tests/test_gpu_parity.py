@@ -575,6 +575,45 @@ def test_codec_bit_exact(lib, O, w, h, c):
 
 # ---- decode from quantized latents ------------------------------------------------------------------
 
+# Order-key spans around what the encoder's candidate search takes (32), where levels coincide
+# (below 16), ordinary ones, and the whole fp16 range.
+@pytest.mark.parametrize("span", [0, 1, 14, 15, 16, 31, 32, 33, 40, 63, 64, 100, 1000, 1024, 5000, 40000, 63487])
+def test_codec_encode_key_spans(lib, O, span):
+    """Blocks whose values' order keys span exactly `span`, from the lowest, the highest and
+    random keys (zero crossings and subnormals among them), the other values at, and one fp32
+    step around, the midpoints of neighbouring levels, on levels and anywhere between: the
+    encoder's bytes equal the oracle's linear scan."""
+    import torch
+    say(f"case: codec key span {span}")
+    rng = np.random.default_rng(span)
+    lo, hi = 0xFFFF - 0xFBFF, 0x8000 + 0x7BFF  # the keys of -65504 and 65504
+
+    def unkey(k):
+        return np.where(k >= 0x8000, k - 0x8000, 0xFFFF - k).astype(np.uint16).view(np.float16).astype(np.float32)
+
+    n, c = 512, 16
+    k0 = np.concatenate([[lo, hi - span, 0x8000 - span // 2, 0x8000 - span, 0x8000, 0x7FFF],
+                         rng.integers(lo, hi - span + 1, n * c - 6)]).clip(lo, hi - span).reshape(n, 1, c)
+    w = (64 * np.arange(16) + 7) // 15
+    lev = unkey(k0 + (span * w[None, :, None] + 32) // 64)  # [block, level, channel]
+    i = rng.integers(0, 15, (n, 16, c))
+    a, b = np.take_along_axis(lev, i, 1), np.take_along_axis(lev, i + 1, 1)
+    mid = ((a.astype(np.float64) + b) / 2).astype(np.float32)
+    kind = rng.integers(0, 5, (n, 16, c))
+    v = np.select([kind == 0, kind == 1, kind == 2, kind == 3],
+                  [mid, np.nextafter(mid, b), np.nextafter(mid, a), a],
+                  (a + (b - a) * rng.uniform(0, 1, (n, 16, c))).astype(np.float32)).astype(np.float32)
+    v[:, 0], v[:, 1] = lev[:, 0], lev[:, 15]
+    vals = np.ascontiguousarray(v.reshape(n, 4, 4, c).transpose(1, 0, 2, 3)).reshape(-1)  # one row of blocks
+    want = np.zeros(n * 12 * c, np.uint8)
+    assert O.ntref_codec_encode(vals.ctypes.data, 4 * n, 4, c, want.ctypes.data) == 0
+    gv = torch.from_numpy(vals).cuda()
+    gb = torch.zeros(want.size, dtype=torch.uint8, device="cuda")
+    nt.check(lib.nt_codec_encode(gv.data_ptr(), 4 * n, 4, c, gb.data_ptr(), None))
+    sync()
+    assert np.array_equal(gb.cpu().numpy(), want)
+
+
 @pytest.mark.parametrize("shape,W,H,jitter,mip_min,mip_max", [
     ("c4", 96, 96, 1.0, 0.0, 3.0),
     ("c4", 100, 37, -1.5, 0.5, 6.0),   # ragged blocks, negative jitter, mips past the last one
