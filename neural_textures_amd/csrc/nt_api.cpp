@@ -494,7 +494,9 @@ void plan16(const nt_params *p, nt_kernel_type type, TrainPlan *plan)
         if (wcols % 16 == 0)
             wcols += 8;
         d.wcols = wcols;
-        const size_t scatter = dx_rows + (random ? (size_t)4 * 32 * G * 4 * 8 : 2 * (size_t)kChunk * wcols * 2);
+        // Random texels: the slots, or (bin order) each wave's weight rows of one pass.
+        const size_t slots = std::max((size_t)4 * 32 * G * 4 * 8, 2 * (size_t)kChunk * kPathStride * 2);
+        const size_t scatter = dx_rows + (random ? slots : 2 * (size_t)kChunk * wcols * 2);
         size_t un = train16_transpose_bytes(plan->shape);
         un = scatter > un ? scatter : un;
         d.group_bytes = (int)((d.tile_bytes + un + 15) & ~(size_t)15);
@@ -1152,7 +1154,10 @@ int train_step_with(const nt_params *p, nt_kernel_type type, void *stream, const
         }
         if (plan.sort_off) {
             // NT_SAMPLES_RANDOM: the slots' samples sorted by bin.
-            e = launch_random_order(random_order_desc(p, plan, ws), s, &d.order);
+            const RandomOrderDesc r = random_order_desc(p, plan, ws);
+            e = launch_random_order(r, s, &d.order);
+            if (e == hipSuccess)
+                e = launch_random_path(r, s);
             if (e != hipSuccess)
                 return hip_status(e, "random-texel sample order");
         }

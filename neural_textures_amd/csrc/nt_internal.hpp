@@ -146,6 +146,17 @@ int random_order_high_bits(int key_bits, int tiles);
 size_t random_order_count_bytes(int n, int key_bits);
 // Bins, then the stable sort; *order is the sorted sample indices (d.vals).
 hipError_t launch_random_order(const RandomOrderDesc &d, hipStream_t s, const uint32_t **order);
+// ... and each tile of kRandomPathTile of its entries (the train kernel's tiles) reordered in
+// place along a path through the bins.
+constexpr int kRandomPathTile = 1024;
+hipError_t launch_random_path(const RandomOrderDesc &d, hipStream_t s);
+
+// The bin-ordered random-texel kernel's scatter: each wave's weight rows (32 samples, hi and
+// lo, kPathCells cells a pass) in rows of kPathStride halves (an odd number of 8-byte chunks:
+// rows fall in distinct LDS banks).
+constexpr int kPathCells = 64;
+constexpr int kPathStride = kPathCells + 4;
+constexpr int kPathMaxCells = 256; // a larger cell box takes per-sample atomics
 
 struct Train16Desc {
     Grid16 grid[NT_MAX_GRIDS];

@@ -974,6 +974,166 @@ __device__ __forceinline__ void gather_records(const Train16Desc &d, float *sbox
     }
 }
 
+// Minimum over each half of the wave (lanes 0-31 and 32-63), left in lanes 0, 16 and 32, 48 as
+// the minima of their rows of 16: four DPP steps within the row (quad permutations, then the
+// half-row and row mirrors).
+__device__ __forceinline__ int row_min(int v)
+{
+    v = min(v, __builtin_amdgcn_update_dpp(v, v, 0xB1, 0xF, 0xF, false));
+    v = min(v, __builtin_amdgcn_update_dpp(v, v, 0x4E, 0xF, 0xF, false));
+    v = min(v, __builtin_amdgcn_update_dpp(v, v, 0x141, 0xF, 0xF, false));
+    v = min(v, __builtin_amdgcn_update_dpp(v, v, 0x140, 0xF, 0xF, false));
+    return v;
+}
+__device__ __forceinline__ int half_min(int rows, int half)
+{
+    return min(__builtin_amdgcn_readlane(rows, 32 * half), __builtin_amdgcn_readlane(rows, 32 * half + 16));
+}
+
+// LDS written by some lanes of a wave is read by others of the same wave: no barrier.
+__device__ __forceinline__ void wave_sync()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// The latent scatter of a wave's 32 random texels in bin order, grid by grid, as the region
+// kernel's MFMA reduction D[cell][ch] = sum_s W[cell][s] dX0[s][ch] with K = the wave's 32
+// samples: the order puts them close together, so their footprints share a small cell box (the
+// box of the 32 footprints, rows padded to a power of two of cells), and each cell that any of
+// them touches takes one 64-byte atomic record instead of one per sample and corner. The cells
+// go through the wave's weight rows kPathCells at a time. A box of more than kPathMaxCells
+// cells (the path jumps at the end of a bin row; few samples an image texel) or a non-finite
+// gradient (whose product with a zero weight is NaN) leaves the grid to per-sample atomics.
+// What bounds the random-texel kernel: before, its atomics (all performed past the L2: 1.07 GB
+// of records for four grids and a million samples, 600 us of 1,127); now the scattered taps
+// (245 us) and the MLP (335 us). Four grids, 1,048,576 samples of 4096^2 texels: 105 records a
+// wave instead of 512, WRITE_SIZE 1,184 -> 373 MB, kernel 1,127 -> 709 us; two grids, 262,144
+// samples of 2048^2: 172 -> 116 us.
+template <int DS, int G>
+__device__ __forceinline__ void scatter_path(const Train16Desc &d, const Grid16 (&own)[G / 2], const _Float16 *dxw,
+                                             _Float16 *wrow, const h8 (&dx0)[G], float u, float v, bool valid, int c,
+                                             int g, int lane)
+{
+    constexpr int J = G / 2;
+    const int i16 = lane & 15, grp = lane >> 4;
+    uint32_t top = 0; // the largest |dX0| bits, two halves
+#pragma unroll
+    for (int q = 0; q < G; ++q)
+#pragma unroll
+        for (int e = 0; e < 8; e += 2) {
+            const h2 p = {dx0[q][e], dx0[q][e + 1]};
+            const uint32_t b = __builtin_bit_cast(uint32_t, p) & 0x7FFF7FFFu;
+            asm("v_pk_max_u16 %0, %1, %2" : "=v"(top) : "v"(top), "v"(b));
+        }
+    const bool finite = __ballot((top & 0xFFFFu) >= 0x7C00u || (top >> 16) >= 0x7C00u) == 0;
+    Footprint f[J];
+    int mnx[J], mny[J], mxx[J], mxy[J]; // row minima of x0, y0, -x0, -y0
+#pragma unroll
+    for (int j = 0; j < J; ++j) {
+        f[j] = bilinear_footprint(u, v, own[j].w, own[j].h, 1.f);
+        constexpr int far = 1 << 30;
+        mnx[j] = row_min(valid ? f[j].x0 : far);
+        mny[j] = row_min(valid ? f[j].y0 : far);
+        mxx[j] = row_min(valid ? -f[j].x0 : far);
+        mxy[j] = row_min(valid ? -f[j].y0 : far);
+    }
+#pragma unroll
+    for (int gi = 0; gi < G; ++gi) {
+        const int j = gi >> 1, half = gi & 1;
+        const int bx = half_min(mnx[j], half), by = half_min(mny[j], half);
+        if (bx == (1 << 30))
+            continue; // no valid sample
+        const int cbw = 2 - half_min(mxx[j], half) - bx, cbh = 2 - half_min(mxy[j], half) - by;
+        const int w = sreg(d.grid[gi].w), h = sreg(d.grid[gi].h);
+        float *grads = sreg(d.grid[gi].grads);
+        const int lg = cbw <= 4 ? 2 : cbw <= 8 ? 3 : cbw <= 16 ? 4 : cbw <= 32 ? 5 : 6;
+        if (!finite || cbw > 64 || cbh > (kPathMaxCells >> lg)) {
+            // Per-sample atomics: corner texels and weights in the weight rows' place, then
+            // lane = 16 corner + channel over the wave's samples.
+            int2 *slots = (int2 *)wrow;
+            wave_sync();
+            if (g == half) {
+#pragma unroll
+                for (int corner = 0; corner < 4; ++corner) {
+                    const int tx = wrap_near(f[j].x0 + (corner & 1), w), ty = wrap_near(f[j].y0 + (corner >> 1), h);
+                    slots[c * 4 + corner] = make_int2(valid ? ty * w + tx : -1, __float_as_int(f[j].w[corner]));
+                }
+            }
+            wave_sync();
+#pragma unroll 4
+            for (int s = 0; s < 32; ++s) {
+                const int2 sl = slots[s * 4 + grp];
+                const float gv = (float)dxw[s * DS + 16 * gi + i16];
+                if (sl.x >= 0 && gv != 0.f)
+                    global_add(grads + (uint32_t)sl.x * 16u + (uint32_t)i16, __int_as_float(sl.y) * gv);
+            }
+            continue;
+        }
+        const int ncell = cbh << lg;
+        const bool inside = bx >= 0 && by >= 0 && bx + cbw <= w && by + cbh <= h;
+        const h8 bv = read_cols8<DS>(dxw, 8 * grp, 16 * gi, i16);
+        _Float16 *rhi = wrow + c * kPathStride, *rlo = rhi + 32 * kPathStride;
+        for (int p = 0; p < ncell; p += kPathCells) {
+            const int nt = (min(ncell - p, kPathCells) + 15) >> 4;
+            // The rows of this pass's tiles cleared (lane group 0: hi, 1: lo), then filled by the
+            // lane group that holds the grid's footprints.
+            wave_sync();
+            uint2 *z = (uint2 *)(g ? rlo : rhi);
+#pragma unroll
+            for (int t = 0; t < kPathCells / 16; ++t)
+                if (t < nt)
+#pragma unroll
+                    for (int k = 0; k < 4; ++k)
+                        z[4 * t + k] = make_uint2(0u, 0u);
+            wave_sync();
+            if (g == half && valid) {
+                const int cell0 = ((f[j].y0 - by) << lg) + (f[j].x0 - bx) - p;
+#pragma unroll
+                for (int corner = 0; corner < 4; ++corner) {
+                    const int cell = cell0 + ((corner >> 1) << lg) + (corner & 1);
+                    if ((unsigned)cell < (unsigned)kPathCells) {
+                        const int k = cell_column(cell);
+                        const _Float16 hi = (_Float16)f[j].w[corner];
+                        rhi[k] = hi;
+                        rlo[k] = (_Float16)(f[j].w[corner] - (float)hi);
+                    }
+                }
+            }
+            wave_sync();
+            f4v acc[kPathCells / 16];
+#pragma unroll
+            for (int t = 0; t < kPathCells / 16; ++t)
+                if (t < nt) {
+                    const _Float16 *a = wrow + (8 * grp + (i16 >> 2)) * kPathStride + 16 * t + 4 * (i16 & 3);
+                    const _Float16 *b = a + 32 * kPathStride;
+                    const h4 h0 = lds_read_tr16(a), h1 = lds_read_tr16(a + 4 * kPathStride);
+                    const h4 l0 = lds_read_tr16(b), l1 = lds_read_tr16(b + 4 * kPathStride);
+                    acc[t] = mfma16(__builtin_shufflevector(h0, h1, 0, 1, 2, 3, 4, 5, 6, 7), bv, (f4v){0.f, 0.f, 0.f, 0.f});
+                    acc[t] = mfma16(__builtin_shufflevector(l0, l1, 0, 1, 2, 3, 4, 5, 6, 7), bv, acc[t]);
+                }
+#pragma unroll
+            for (int t = 0; t < kPathCells / 16; ++t)
+                if (t < nt) {
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        // D row 4 grp + r holds cell 16 t + 4 r + grp of the pass (cell_column).
+                        const int cell = p + 16 * t + 4 * r + grp;
+                        const int cx = cell & ((1 << lg) - 1), cy = cell >> lg;
+                        int tx = bx + cx, ty = by + cy;
+                        if (!inside) {
+                            tx = wrap_near(tx, w);
+                            ty = wrap_near(ty, h);
+                        }
+                        if (cx < cbw && cy < cbh && acc[t][r] != 0.f)
+                            global_add(grads + ((uint32_t)(ty * w + tx) * 16u + (uint32_t)i16), acc[t][r]);
+                    }
+                }
+        }
+    }
+}
+
 // dW slots per round of the end-of-kernel handoff between the two groups: all of them,
 // except for the 4-grid network (random texels), whose group regions hold two.
 template <class S>
@@ -1339,7 +1499,11 @@ __global__ __launch_bounds__(kTrainThreads *NG) void train16_kernel(Train16Desc 
         // to fp32 rounding) goes straight to global memory, all C channels read back from
         // the dX0 row.
         store_rows<KQ0, dx_stride(S::K0)>(dxs, dx0, col, g);
-        if constexpr (RND) {
+        if constexpr (RND && ORD) {
+            // Bin order: only the wave's own rows are read and written, so no barrier.
+            scatter_path<dx_stride(S::K0), G>(d, own, dxs + 32 * wave * dx_stride(S::K0),
+                                              whi + wave * (64 * kPathStride), dx0, u, v, valid, c, g, lane);
+        } else if constexpr (RND) {
             // Random texels: no two samples of a chunk are expected to share a texel, so each
             // sample's corners go straight to the gradients (train.cu:460-509's per-sample
             // atomics). The wave's lanes record each (sample, grid) corner's texel and weight

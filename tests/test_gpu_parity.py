@@ -285,6 +285,47 @@ def test_train_step_random_texels(lib, O, shape, region, max_wg, flags, image):
     check_train_grads(st, gs, alt)
 
 
+@pytest.mark.parametrize("shape,image,n,overflow", [
+    # few texels: every wave's box is small and the cells are shared by many samples; wraps
+    ("c2", 16, 3000, False), ("c4", 64, 2100, False),
+    # one sample to 1,024 texels: boxes past 64 cells (several passes) and past 256 (atomics)
+    ("c2", 1024, 1100, False), ("c4", 512, 1030, False),
+    # a partial wave, one sample alone, one past a tile
+    ("c2", 128, 33, False), ("c4", 128, 1, False), ("c2", 128, 1025, False),
+    # gradients past fp16: only the corners a non-finite sample reaches become non-finite
+    ("c2", 64, 1500, True),
+])
+def test_random_texel_path_scatter(lib, O, shape, image, n, overflow):
+    """The bin-ordered random-texel scatter (each wave's cell box reduced on the matrix cores)
+    against the oracle's per-sample sums, at the sizes where its passes change."""
+    say(f"case: path scatter {shape} image {image} samples {n} overflow {overflow}")
+    st = make_state(shape, image=image, region=(n, 1), seed=31)
+    st.sample_mode = abi.NT_SAMPLES_RANDOM
+    if overflow:  # a texel of one texture far past the others: a few samples' gradients overflow
+        t = st.textures[0].texels.reshape(image, image, 4)
+        t[5, 9, 0] = 3e30
+    alt = st.converted(False)
+    gs = st.to_torch()
+    oracle_step(O, st, 0)
+    oracle_step(O, alt, 0, accum_f32=True)
+    nt.check(lib.nt_set_test_hooks(0, abi.NT_HOOK_SORT_RANDOM))
+    try:
+        gs = gpu_workspace(lib, gs, 0)
+        nt.check(lib.nt_train_step(C.byref(gs.params()), 0, None))
+        sync()
+    finally:
+        nt.check(lib.nt_set_test_hooks(0, 0))
+    if not overflow:
+        check_train_grads(st, gs, alt)
+        return
+    for h, g in zip(st.grids, gs.grids):
+        got = to_np(g.grads)
+        assert not np.all(np.isfinite(h.grads)) and np.any(np.isfinite(h.grads) & (h.grads != 0))
+        assert np.array_equal(np.isfinite(got), np.isfinite(h.grads))
+        fine = np.isfinite(got)
+        assert_close(got[fine], h.grads[fine], "finite latent gradients")
+
+
 def test_random_texel_sorted_step_is_deterministic(lib):
     """The bin sort of NT_SAMPLES_RANDOM is stable, so a step's slots hold the same samples
     on every run and the network gradient (summed per workgroup in slot order, then in a
