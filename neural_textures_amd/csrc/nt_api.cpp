@@ -427,21 +427,42 @@ void plan16(const nt_params *p, nt_kernel_type type, TrainPlan *plan)
     d.ntex = p->num_textures;
     const int rw = p->region_width > 0 ? p->region_width : NT_DEFAULT_REGION;
     const int rows = (int)(((int64_t)p->num_samples + rw - 1) / rw);
-    // Region: tiles of 64 x 8NG positions. Random texels: tiles of 512 consecutive samples
-    // (of the position-sorted order).
-    d.tiles_x = random ? 1 : (rw + 4 * kChunkW - 1) / (4 * kChunkW);
-    const int64_t tiles_y = random ? ((int64_t)p->num_samples + 4 * kChunk * NG - 1) / (4 * kChunk * NG)
-                                   : (rows + kChunkH * NG - 1) / (kChunkH * NG);
-    if ((int64_t)d.tiles_x * tiles_y > (1 << 30))
-        return;
+    // Region: tiles of 16 tile_chunks x 8NG positions. Random texels: tiles of 512 NG consecutive
+    // samples (of the bin order).
     // One workgroup per CU (the kernel's registers and LDS allow no second one); each takes
     // every nwg-th tile, so that fewer, longer-lived workgroups stage the weights and write
     // MLP-gradient partials.
     // A test hook can lower the cap (to give workgroups several tiles at small sizes).
-    d.ntiles = d.tiles_x * tiles_y;
     int cap = device_cu_count();
     if (const int hook = g_hook_max_workgroups.load(std::memory_order_relaxed); hook > 0)
         cap = std::min(cap, hook);
+    // A workgroup's time is its chunks in sequence, so a tile has four chunks, or two or one
+    // where that leaves the busiest workgroup fewer of them: whole steps of two grids at 64 x 32
+    // samples 44.8 -> 21.5 us and at 300 x 217 48.5 -> 32.9 us (one chunk a workgroup, then
+    // two); the reference network at 509 x 331, 168 tiles of four on 256 CUs, 76.8 -> 69.2 us
+    // (three). Equal counts keep the wider tile (fewer halo texels and box flushes).
+    d.tile_chunks = 4;
+    if (random) {
+        d.tiles_x = 1;
+        const int64_t n = ((int64_t)p->num_samples + 4 * kChunk * NG - 1) / (4 * kChunk * NG);
+        if (n > (1 << 30))
+            return;
+        d.ntiles = (int)n;
+    } else {
+        int64_t best = 0;
+        for (int tc = 4; tc >= 1; tc /= 2) {
+            const int64_t tx = (rw + tc * kChunkW - 1) / (tc * kChunkW), n = tx * ((rows + kChunkH * NG - 1) / (kChunkH * NG));
+            const int64_t serial = (n + cap - 1) / cap * tc;
+            if (n > (1 << 30) || (best > 0 && serial >= best))
+                continue;
+            best = serial;
+            d.tile_chunks = tc;
+            d.tiles_x = (int)tx;
+            d.ntiles = (int)n;
+        }
+        if (best == 0)
+            return;
+    }
     d.nwg = std::min(d.ntiles, cap);
     d.xcd_per = (d.ntiles % 8 == 0 && d.nwg % 8 == 0) ? d.ntiles / 8 : 0;
     // Margin of the chunk cell box beyond the cells positions can reach. A test hook drops
@@ -538,7 +559,7 @@ void plan16(const nt_params *p, nt_kernel_type type, TrainPlan *plan)
         q.gk = 0;
         if (!c3 || random || q.ncell > 0)
             continue;
-        const int bw = (int)std::ceil(4 * kChunkW * (double)q.w / p->image_width) + 4;
+        const int bw = (int)std::ceil(d.tile_chunks * kChunkW * (double)q.w / p->image_width) + 4;
         const int bh = (int)std::ceil(kChunkH * NG * (double)q.h / p->image_height) + 4;
         if ((size_t)d.box_lds_off + ((size_t)d.box_floats + (size_t)bw * bh * C) * 4 > kMaxLds)
             continue;

@@ -174,6 +174,7 @@ struct Train16Desc {
     // 1/image_w, 1/image_h, 1/num_samples where that is a power of two (a product with the
     // reciprocal then equals the quotient exactly), else 0 (divide).
     float inv_w, inv_h, inv_samples;
+    int tile_chunks; // region: 16-position chunks across a tile (1, 2 or 4)
     int tiles_x, ntiles, nwg, xcd_per; // xcd_per > 0: workgroups of one XCD take consecutive tiles
     int group_off, group_bytes, tile_bytes; // per 4-wave group: target tile, then the union
     int wcols;                              // halves per scatter-weight row (one row per sample)

@@ -5,8 +5,9 @@
 //
 // A workgroup is NG groups of four waves (NG = 2 for the 2-grid network: two waves per
 // SIMD, so one wave's LDS and memory latency hides behind the other's work). It owns a
-// 64 x 8NG block of region positions; group gr walks rows [8gr, 8gr + 8) as four 16 x 8
-// chunks of 128 samples, one 32-sample MFMA tile per wave. Per chunk:
+// 64 x 8NG block of region positions (narrower where that spreads a small region over more
+// workgroups); group gr walks rows [8gr, 8gr + 8) as four (two, one) 16 x 8 chunks of 128
+// samples, one 32-sample MFMA tile per wave. Per chunk:
 //   - the group's Catmull-Rom target tile is copied into its LDS region by DMA
 //     (global_load_lds) at the chunk start and published after the forward pass, so the
 //     loads overlap sampling and MLP;
@@ -1142,9 +1143,13 @@ constexpr int handoff_slots()
     return S::K0 == 64 ? 2 : T16Layout<S, 1>::slots;
 }
 
-template <class S, int C, int NG, bool RND, bool ORD = false>
+// ALT: random texels, slots read in bin order (ORD); region, tiles of d.tile_chunks chunks
+// instead of four (NARROW; its own kernel, as a loop bound read at run time costs the
+// four-chunk one 1.7 % with four grids).
+template <class S, int C, int NG, bool RND, bool ALT = false>
 __global__ __launch_bounds__(kTrainThreads *NG) void train16_kernel(Train16Desc d)
 {
+    constexpr bool ORD = RND && ALT, NARROW = !RND && ALT;
     static_assert(!RND || C == 16, "random texels are built for 16-channel grids");
     using LY = T16Layout<S, NG>;
     // Grids: one per 16 inputs with 16 channels; the 3-channel network has four.
@@ -1178,7 +1183,7 @@ __global__ __launch_bounds__(kTrainThreads *NG) void train16_kernel(Train16Desc 
         int b = b0;
         if (d.xcd_per > 0)
             b = (b & 7) * d.xcd_per + (b >> 3); // the workgroups of one XCD share an L2: give them neighbouring tiles
-        tx0 = (b % d.tiles_x) * (kChunkW * 4);
+        tx0 = (b % d.tiles_x) * (kChunkW * (NARROW ? d.tile_chunks : 4));
         ty0 = (b / d.tiles_x) * (kChunkH * NG);
         return b;
     };
@@ -1325,7 +1330,8 @@ __global__ __launch_bounds__(kTrainThreads *NG) void train16_kernel(Train16Desc 
         }
     }
 
-    for (int chunk = 0; chunk < 4; ++chunk) {
+    const int nchunk = NARROW ? d.tile_chunks : 4;
+    for (int chunk = 0; chunk < nchunk; ++chunk) {
         const int cx0 = d.off_x + tx0 + chunk * kChunkW, cy0 = d.off_y + ty0 + kChunkH * gr;
         // With gather boxes both copies are untracked: the gather's LDS reads (another buffer)
         // then wait for neither.
@@ -1391,7 +1397,7 @@ __global__ __launch_bounds__(kTrainThreads *NG) void train16_kernel(Train16Desc 
         if constexpr (GBOX) {
             if (d.gbox_off != 0) {
                 float4 *gnext = gbox + ((gq + 1) & 1) * gbox_step;
-                if (chunk < 3) {
+                if (chunk + 1 < nchunk) {
                     gbox_fetch_async(gl, gnext, cx0 + kChunkW, cy0, wave);
                 } else if (b0 + (int)gridDim.x < d.ntiles) {
                     int nx0, ny0;
@@ -1934,10 +1940,10 @@ using ShapeRef = Shape<16, 32, 2>;
 using ShapeC2 = Shape<32, 64, 2>;
 using ShapeC4 = Shape<64, 64, 3>;
 
-template <class S, int C, int NG, bool RND, bool ORD = false>
+template <class S, int C, int NG, bool RND, bool ALT = false>
 static hipError_t launch16(const Train16Desc &d, size_t lds, hipStream_t s)
 {
-    auto k = train16_kernel<S, C, NG, RND, ORD>;
+    auto k = train16_kernel<S, C, NG, RND, ALT>;
     // Raise the kernel's dynamic LDS limit to the whole 160 KB once (thread-safe).
     static std::once_flag once;
     static hipError_t configured = hipSuccess;
@@ -2024,17 +2030,21 @@ size_t train16_transpose_bytes(int shape)
     return shape == kShapeRef || shape == kShapeC2 || shape == kShapeC4 ? 2 * kChunk * kFeatStride * 2 : 0;
 }
 
+template <class S, int C, int NG>
+static hipError_t launch_region(const Train16Desc &d, size_t lds, hipStream_t s)
+{
+    return d.tile_chunks == 4 ? launch16<S, C, NG, false>(d, lds, s) : launch16<S, C, NG, false, true>(d, lds, s);
+}
+
 hipError_t launch_train16(int shape, const Train16Desc &d, size_t lds, hipStream_t s)
 {
     switch (shape) {
     case kShapeRef:
-        return d.random_texels ? hipErrorInvalidValue : launch16<ShapeRef, 3, 2, false>(d, lds, s);
+        return d.random_texels ? hipErrorInvalidValue : launch_region<ShapeRef, 3, 2>(d, lds, s);
     case kShapeC2:
-        return d.random_texels ? launch_train16_random(shape, d, lds, s)
-                               : launch16<ShapeC2, 16, 2, false>(d, lds, s);
+        return d.random_texels ? launch_train16_random(shape, d, lds, s) : launch_region<ShapeC2, 16, 2>(d, lds, s);
     case kShapeC4:
-        return d.random_texels ? launch_train16_random(shape, d, lds, s)
-                               : launch16<ShapeC4, 16, 1, false>(d, lds, s);
+        return d.random_texels ? launch_train16_random(shape, d, lds, s) : launch_region<ShapeC4, 16, 1>(d, lds, s);
     default:
         return hipErrorInvalidValue;
     }

@@ -252,6 +252,24 @@ def test_train_step_scatter_out_of_box_paths(lib, O, shape):
     check_train_grads(st, gs, alt, biases=False)
 
 
+@pytest.mark.parametrize("shape,rows", [("c2", 16), ("c4", 8), ("ref16", 16), ("ref16f", 16)])
+@pytest.mark.parametrize("max_wg,ragged", [(1, 0), (4, 0), (0, 0), (1, 5), (4, 5), (0, 5), (3, 37)],
+                         ids=["four-chunks", "two-chunks", "one-chunk", "four-chunks-ragged", "two-chunks-ragged",
+                              "one-chunk-ragged", "one-chunk-looping-ragged"])
+def test_train_step_tile_widths(lib, O, shape, rows, max_wg, ragged):
+    """A region of eight chunk columns and one tile row (ragged: that many columns narrower and
+    one row shorter) over one, three, four and enough workgroups: tiles of four, two and one
+    chunks, the one that leaves the busiest workgroup the fewest. Gradients match the oracle's."""
+    say(f"case: tile widths {shape} workgroups {max_wg} ragged {ragged}")
+    nt.check(lib.nt_set_test_hooks(max_wg, 0))
+    try:
+        st, gs, alt = run_train_pair(lib, O, shape, 256, (128 - ragged, rows - (ragged > 0)), (21, 240 if ragged else 7),
+                                     abi.NT_UNCONSTRAINED, seed=3)
+    finally:
+        nt.check(lib.nt_set_test_hooks(0, 0))
+    check_train_grads(st, gs, alt)
+
+
 @pytest.mark.parametrize("shape,region,max_wg,flags,image", [
     ("ref", (64, 32), 0, 0, 128), ("c1", (64, 32), 0, 0, 128), ("c2", (64, 32), 0, 0, 128),
     ("c4", (64, 32), 0, 0, 128), ("c2", (50, 13), 2, 0, 128), ("c4", (100, 7), 1, 0, 128),
