@@ -1772,14 +1772,18 @@ int nt_forward(const nt_latents *latents, const nt_mlp *mlp, nt_filter filter, c
         return st;
     if (count == 0)
         return ok();
-    d.count = count;
-    d.uvz = uvz;
-    d.features = features;
-    d.out16 = outputs;
-    d.out_stride = mlp->sizes[mlp->num_layers];
-    const int mode = filter == NT_FILTER_BILINEAR ? kFwdBilinear : kFwdCatmullRom;
+    SampleDesc q{};
+    q.mlp = d.mlp;
+    q.G = d.G;
+    for (int gi = 0; gi < NT_MAX_GRIDS; ++gi)
+        q.grid[gi] = d.grid[gi < d.G ? gi : 0];
+    q.count = count;
+    q.uvz = uvz;
+    q.features = features;
+    q.out16 = outputs;
+    q.out_stride = mlp->sizes[mlp->num_layers];
     ProfileScope prof((hipStream_t)stream);
-    return hip_status(launch_forward(shape, mode, d, (hipStream_t)stream), "forward launch");
+    return hip_status(launch_sample(shape, filter == NT_FILTER_CATMULL_ROM, q, (hipStream_t)stream), "forward launch");
 }
 
 int nt_bc6_init(const nt_latents *lat, void *stream)

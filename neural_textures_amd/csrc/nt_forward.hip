@@ -1,7 +1,7 @@
 // nt_forward.hip — forward-only passes on gfx950: the tiny-MLP forward
-// (mlp.h:18-99, the path tests/forward_pass_test.cu exercises), latent sample + MLP at
-// given coordinates, full-image inference (train.cu:917-961) and decode from
-// codec-quantized latents.
+// (mlp.h:18-99, the path tests/forward_pass_test.cu exercises), full-image inference
+// (train.cu:917-961) where nt_infer.hip does not apply, and decode from codec-quantized
+// latents.
 //
 // Each wave runs 32-sample MFMA tiles in a grid-stride loop; forward weight fragments are
 // staged in LDS once per workgroup. Lane group g of sample c (lane = 32g + c) gathers the
@@ -98,43 +98,6 @@ __device__ __forceinline__ void sample_bilinear(const FwdDesc &d, float u, float
                 x[q][e] = a;
             }
         }
-    }
-}
-
-// 16-tap Catmull-Rom latent sample on mip 0: fp32 accumulation, one fp16 rounding.
-template <int C, int KQ>
-__device__ __forceinline__ void sample_catmull_rom(const FwdDesc &d, float u, float v, int g,
-                                                   h8 (&x)[KQ])
-{
-#pragma unroll
-    for (int q = 0; q < KQ; ++q) {
-        float acc[8];
-#pragma unroll
-        for (int e = 0; e < 8; ++e)
-            acc[e] = 0.f;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-            const int feat = 16 * q + 8 * g + e;
-            if (feat >= d.G * C)
-                continue;
-            const GridDesc &gr = d.grid[feat / C];
-            const int ch = feat % C;
-            float wx[4], wy[4];
-            const int x0 = cr_axis(u, gr.w, wx);
-            const int y0 = cr_axis(v, gr.h, wy);
-            const float *vals = gr.values + gr.mip_off[0] * C;
-            for (int j = 0; j < 4; ++j) {
-                const int ty = wrap_coord(y0 + j, gr.h);
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const int tx = wrap_coord(x0 + i, gr.w);
-                    acc[e] = fmaf(vals[((int64_t)ty * gr.w + tx) * C + ch], wx[i] * wy[j], acc[e]);
-                }
-            }
-        }
-#pragma unroll
-        for (int e = 0; e < 8; ++e)
-            x[q][e] = (_Float16)acc[e];
     }
 }
 
@@ -312,15 +275,6 @@ __global__ __launch_bounds__(kFwdThreads, fwd_min_blocks<MODE>()) void forward_k
                     x0[q][e] = (valid && feat < in) ? bits_h(d.inputs[(int64_t)s * in + feat])
                                                     : (_Float16)0.f;
                 }
-        } else if constexpr (MODE == kFwdBilinear || MODE == kFwdCatmullRom) {
-            const int sc = valid ? s : 0;
-            u = d.uvz[3 * (int64_t)sc];
-            v = d.uvz[3 * (int64_t)sc + 1];
-            const float z = d.uvz[3 * (int64_t)sc + 2];
-            if constexpr (MODE == kFwdBilinear)
-                sample_bilinear<C, KQ0>(d, u, v, z, g, x0);
-            else
-                sample_catmull_rom<C, KQ0>(d, u, v, g, x0);
         } else if constexpr (MODE == kFwdInference) {
             const int sc = valid ? s : 0;
             const int px = sc % d.image_w, py = sc / d.image_w;
@@ -344,18 +298,6 @@ __global__ __launch_bounds__(kFwdThreads, fwd_min_blocks<MODE>()) void forward_k
             else
                 sample_codec<C, KQ0>(d, u, v, z, g, x0);
         }
-        if (d.features != nullptr && valid) {
-            const int nf = d.G * C;
-#pragma unroll
-            for (int q = 0; q < KQ0; ++q)
-#pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    const int feat = natural_feature(q, g, e);
-                    if (feat < nf)
-                        d.features[(int64_t)s * nf + feat] = h_bits(x0[q][e]);
-                }
-        }
-
         // MLP forward (mlp.h:65-99)
         h8 xh[HQ];
         {
@@ -766,10 +708,6 @@ template <class S, int C>
 static hipError_t launch_modes(int mode, const FwdDesc &d, hipStream_t s)
 {
     switch (mode) {
-    case kFwdBilinear:
-        return launch_fwd<S, C, kFwdBilinear>(d, s);
-    case kFwdCatmullRom:
-        return launch_fwd<S, C, kFwdCatmullRom>(d, s);
     case kFwdInference:
         return launch_fwd<S, C, kFwdInference>(d, s);
     case kFwdDecode:

@@ -51,10 +51,6 @@ struct InferLayout {
     static constexpr int bytes = frag_bytes + bias_bytes + kFwdWaves * 32 * kPixelStride * 4;
 };
 
-// Grids a lane samples: 16 and 3 channels, grids g and g + 2; 8 channels, grid g.
-template <int C>
-constexpr int lane_grids() { return C == 8 ? 1 : 2; }
-
 } // namespace
 
 // NT: textures per lane (textures g and g + 2): 1 for up to two textures, else 2.
@@ -62,7 +58,8 @@ template <class S, int C, int NT>
 __global__ __launch_bounds__(kFwdThreads, 2) void inference_kernel(InferDesc d)
 {
     constexpr int L = S::L, NH = S::NH, KQ0 = S::K0 / 16, HQ = S::H / 16, HA = S::t32(S::H);
-    constexpr int NG = C == 16 ? KQ0 / 2 : lane_grids<C>(); // grids per lane
+    // Grids per lane: 16 and 3 channels, grids g and g + 2; 8 channels, four channels of both.
+    constexpr int NG = C == 16 ? KQ0 / 2 : 2;
     using LY = InferLayout<S>;
     extern __shared__ __align__(16) unsigned char smem[];
     h8 *frags = (h8 *)smem;
@@ -78,11 +75,11 @@ __global__ __launch_bounds__(kFwdThreads, 2) void inference_kernel(InferDesc d)
     bool on[NG];
 #pragma unroll
     for (int j = 0; j < NG; ++j) {
-        const InferGrid &a = d.grid[2 * j], &b = d.grid[2 * j + 1];
-        vals[j] = g ? sreg(b.values) : sreg(a.values);
+        const InferGrid &a = d.grid[C == 8 ? j : 2 * j], &b = d.grid[C == 8 ? j : 2 * j + 1];
+        vals[j] = g ? sreg(b.values) + (C == 8 ? 4 : 0) : sreg(a.values);
         gw[j] = g ? sreg(b.w) : sreg(a.w);
         gh[j] = g ? sreg(b.h) : sreg(a.h);
-        on[j] = 2 * j + g < d.G;
+        on[j] = (C == 8 ? j : 2 * j + g) < d.G;
     }
     const float4 *tex[NT];
     int nch[NT], out0[NT];
@@ -157,7 +154,7 @@ __global__ __launch_bounds__(kFwdThreads, 2) void inference_kernel(InferDesc d)
 #pragma unroll
             for (int q = 0; q < KQ0; ++q)
                 x0[q] = (h8)(_Float16)0.f;
-            constexpr int F4 = C == 3 ? 1 : C / 4;
+            constexpr int F4 = C == 16 ? 4 : 1;
             using Texel = typename std::conditional<C == 3, f3, float4>::type;
             Texel tx[NG][4][F4];
             float wgt[NG][4];
@@ -179,7 +176,7 @@ __global__ __launch_bounds__(kFwdThreads, 2) void inference_kernel(InferDesc d)
                     } else {
 #pragma unroll
                         for (int i = 0; i < F4; ++i)
-                            tx[j][k][i] = load_global((const float4 *)vals[j] + (at[k] * (uint32_t)F4 + (uint32_t)i));
+                            tx[j][k][i] = load_global((const float4 *)vals[j] + (at[k] * (uint32_t)(C / 4) + (uint32_t)i));
                     }
                 }
             }
@@ -207,6 +204,22 @@ __global__ __launch_bounds__(kFwdThreads, 2) void inference_kernel(InferDesc d)
                     x0[0][3 * j + 1] = on[j] ? a01[j][1] : (_Float16)0.f;
                     x0[0][3 * j + 2] = on[j] ? a2[j] : (_Float16)0.f;
                 }
+            } else if constexpr (C == 8) {
+#pragma unroll
+                for (int j = 0; j < NG; ++j) {
+                    h4 a = {(_Float16)0.f, (_Float16)0.f, (_Float16)0.f, (_Float16)0.f};
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) {
+                        const float4 &t = tx[j][k][0];
+                        const float w = wgt[j][k];
+                        const f2 p0 = {rn32(w * t.x), rn32(w * t.y)}, p1 = {rn32(w * t.z), rn32(w * t.w)};
+                        a = a + __builtin_shufflevector(__builtin_convertvector(p0, h2), __builtin_convertvector(p1, h2), 0, 1,
+                                                        2, 3);
+                    }
+#pragma unroll
+                    for (int ch = 0; ch < 4; ++ch)
+                        x0[0][4 * j + ch] = on[j] ? a[ch] : (_Float16)0.f;
+                }
             } else {
 #pragma unroll
                 for (int j = 0; j < NG; ++j)
@@ -216,7 +229,7 @@ __global__ __launch_bounds__(kFwdThreads, 2) void inference_kernel(InferDesc d)
 #pragma unroll
                         for (int k = 0; k < 4; ++k)
                             a = accumulate_products(a, wgt[j][k], tx[j][k][i], tx[j][k][i + 1]);
-                        x0[(C == 16 ? 2 * j : 0) + i / 2] = on[j] ? a : (h8)(_Float16)0.f;
+                        x0[2 * j + i / 2] = on[j] ? a : (h8)(_Float16)0.f;
                     }
             }
 

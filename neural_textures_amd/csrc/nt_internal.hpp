@@ -247,8 +247,6 @@ struct ReduceDesc {
 
 enum FwdMode {
     kFwdMlp = 0,
-    kFwdBilinear = 1,
-    kFwdCatmullRom = 2,
     kFwdInference = 3,
     kFwdDecode = 4,   // samples codec blocks directly
     kFwdDecode16 = 5  // samples the fp16 texels of the first decode pass
@@ -345,7 +343,7 @@ inline int forward_blocks(int count)
     return blocks < 1 ? 1 : (blocks > kFwdMaxBlocks ? kFwdMaxBlocks : blocks);
 }
 
-// Forward-only passes: nt_mlp_forward, nt_forward, nt_inference, nt_decode.
+// Forward-only passes: nt_mlp_forward, nt_inference, nt_decode.
 struct FwdDesc {
     MlpDesc mlp;
     GridDesc grid[NT_MAX_GRIDS];
@@ -359,8 +357,6 @@ struct FwdDesc {
     float inv_w, inv_h; // 1/image_w, 1/image_h when powers of two (exact), else 0 (divide)
     const uint16_t *half_values[NT_MAX_GRIDS]; // kFwdDecode16: expanded fp16 texel chains
     const uint16_t *inputs; // kFwdMlp
-    const float *uvz;       // kFwdBilinear / kFwdCatmullRom
-    uint16_t *features;     // optional fp16 features
     uint16_t *out16;        // fp16 outputs
     float *out32;           // kFwdInference
     float *sse;             // kFwdInference
@@ -368,6 +364,17 @@ struct FwdDesc {
     int out_stride;         // outputs per sample
     uint32_t seed;
     float jitter, mip_min, mip_max;
+};
+
+// Latent sample + MLP at given coordinates (nt_sample.hip).
+struct SampleDesc {
+    MlpDesc mlp;
+    GridDesc grid[NT_MAX_GRIDS]; // entries past G repeat grid 0
+    int G, count;
+    const float *uvz;
+    uint16_t *features; // optional fp16 features [count][G * C]
+    uint16_t *out16;
+    int out_stride;
 };
 
 // Full-image inference with reference textures of the image's size (nt_infer.hip): strips of
@@ -480,6 +487,7 @@ __host__ __device__ inline int box_last(int b1, int image, float jitter, int lev
 }
 hipError_t launch_decode_box(int shape, const DecodeBoxDesc &d, hipStream_t s);
 size_t decode_box_weight_bytes(int shape);
+hipError_t launch_sample(int shape, bool catmull_rom, const SampleDesc &d, hipStream_t s);
 hipError_t launch_inference(int shape, const InferDesc &d, hipStream_t s);
 // *sse += the sum of partial[0..n) in a fixed order (one workgroup).
 hipError_t launch_sse_reduce(const float *partial, int n, float *sse, hipStream_t s);

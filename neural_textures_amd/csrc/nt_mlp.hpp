@@ -146,7 +146,8 @@ __device__ h8 weight_fragment(const MlpDesc &m, int idx)
 // per fragment). 3 channels (up to four grids, one k-step): lane group g holds grid g's
 // channels (e = 0..2), grid g + 2's (e = 3..5) and two of the padding features 12..15
 // (e = 6, 7), so that each lane samples two grids and the two groups together cover all
-// sixteen inputs. 8 channels (up to two grids): grid g's channels, the natural order.
+// sixteen inputs. 8 channels (up to two grids): channels 4g .. 4g + 3 of grid 0 (e = 0..3) and
+// of grid 1 (e = 4..7), the chained order, so that one grid occupies both lane groups.
 template <int C>
 __host__ __device__ constexpr int input_feature(int q, int g, int e)
 {
@@ -155,12 +156,12 @@ __host__ __device__ constexpr int input_feature(int q, int g, int e)
     else if constexpr (C == 3)
         return e < 3 ? 3 * g + e : e < 6 ? 3 * (g + 2) + (e - 3) : 12 + 2 * g + (e - 6);
     else
-        return 16 * q + 8 * g + e;
+        return 16 * q + 8 * (e >> 2) + 4 * g + (e & 3);
 }
 
 // Layer l's forward fragments, items tid, tid + NT, ... (an item is a fragment's lane): a
-// lane's eight inputs of one output row are 16 consecutive bytes of the weight row (layer 0;
-// with 3 channels eight scattered halves) or two runs of 8 bytes (chained order), so the
+// lane's eight inputs of one output row are 16 consecutive bytes of the weight row (layer 0
+// with 16 channels; with 3 eight scattered halves) or two runs of 8 bytes (chained order), so the
 // fragments are read with those loads, all of them issued before the first LDS store.
 template <class S, int C, int l, int NT>
 __device__ __forceinline__ void stage_forward_layer(const MlpDesc &m, h8 *frags, int tid)
@@ -175,7 +176,7 @@ __device__ __forceinline__ void stage_forward_layer(const MlpDesc &m, h8 *frags,
         const int c = lane & 31, g = lane >> 5, a = f / qn, q = f % qn;
         const int n = 32 * a + c;
         const uint16_t *row = W + min(n, kout - 1) * kin;
-        if constexpr (l > 0) {
+        if constexpr (l > 0 || C == 8) {
             const uint2 lo = load_global((const uint2 *)(row + chained_feature(q, g, 0)));
             const uint2 hi = load_global((const uint2 *)(row + chained_feature(q, g, 4)));
             v[j] = __builtin_bit_cast(h8, make_uint4(lo.x, lo.y, hi.x, hi.y));

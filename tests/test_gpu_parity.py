@@ -15,7 +15,7 @@ import pytest
 
 import neural_textures_amd as nt
 from neural_textures_amd import abi, params as P
-from helpers import assert_close, make_state, oracle_step, rel_err, to_np, gpu_workspace
+from helpers import SHAPES, assert_close, make_state, oracle_step, rel_err, to_np, gpu_workspace
 from oracle_lib import load_oracle
 
 pytestmark = pytest.mark.gpu
@@ -124,6 +124,58 @@ def test_forward_features_bit_exact(lib, O, shape, filt):
     assert np.array_equal(gf.cpu().numpy().view(np.uint16), feats)
     got = go.cpu().numpy().view(np.float16).astype(np.float32)
     assert_close(got, outs.view(np.float16).astype(np.float32), "outputs")
+
+
+@pytest.mark.parametrize("shape,grids", [("ref", 4), ("ref", 2), ("c1", 1), ("c1", 2), ("c2", 2), ("c4", 4)])
+@pytest.mark.parametrize("filt", [abi.NT_FILTER_BILINEAR, abi.NT_FILTER_CATMULL_ROM])
+@pytest.mark.parametrize("n,shift", [(1, 0), (31, 0), (33, 1), (300, 0)])
+def test_forward_coordinates_and_sizes(lib, O, shape, grids, filt, n, shift):
+    """nt_forward's sampled features bit for bit: partial tiles, fewer grids than the network's
+    padding, one- and two-grid 8-channel networks, coordinates many grids outside [0, 1] and mip
+    coordinates past both ends, grids down to one texel, weights off 16-byte alignment."""
+    import torch
+    say(f"case: forward {shape} grids {grids} filter {filt} n {n} weights off by {shift} halves")
+    cfg = SHAPES[shape]
+    rng = np.random.default_rng(n + grids)
+    sizes = [(33, 20, 4), (7, 9, 3), (4, 1, 1), (1, 2, 2)][:grids]
+    gs_ = [P.make_grid(w, h, m, cfg["C"], rng, with_adam=False) for w, h, m in sizes]
+    net = P.make_network([grids * cfg["C"]] + cfg["sizes"][1:], rng=rng, init="xavier")
+    for l in range(net.num_layers):
+        net.biases[l] = P.f16_bits(rng.uniform(-0.1, 0.1, net.sizes[l + 1]))
+    uvz = rng.uniform(-0.1, 1.1, size=(n, 3)).astype(np.float32)
+    uvz[n // 2:, :2] = rng.uniform(-9, 9, size=(n - n // 2, 2))
+    uvz[:, 2] = rng.uniform(-1.5, 5.5, n) if filt == abi.NT_FILTER_BILINEAR else 0.0
+    uvz[0] = [0.0, 1.0, 1.0]
+
+    def latents(gg):
+        lat = abi.nt_latents()
+        lat.num_grids, lat.channels = len(gg), cfg["C"]
+        for i, g in enumerate(gg):
+            lat.grids[i] = g.struct()
+        return lat
+
+    F, no = net.sizes[0], net.sizes[-1]
+    feats, outs = np.zeros(n * F, np.uint16), np.zeros(n * no, np.uint16)
+    assert O.ntref_forward(C.byref(latents(gs_)), C.byref(net.struct()), filt, uvz.ctypes.data, n,
+                           feats.ctypes.data, outs.ctypes.data) == 0
+    gg = [g.converted(True, "cuda") for g in gs_]
+    gnet = net.converted(True, "cuda")
+    for l in range(net.num_layers):
+        w = torch.zeros(gnet.weights[l].numel() + shift, dtype=torch.int16, device="cuda")
+        w[shift:] = gnet.weights[l].view(torch.int16)
+        gnet.weights[l] = w[shift:]
+    guvz = torch.from_numpy(uvz).cuda()
+    gf = torch.zeros(n * F, dtype=torch.int16, device="cuda")
+    go = torch.zeros(n * no, dtype=torch.int16, device="cuda")
+    lat = latents(gg)
+    for features in (gf.data_ptr(), None):
+        go.zero_()
+        nt.check(lib.nt_forward(C.byref(lat), C.byref(gnet.struct()), filt, guvz.data_ptr(), n, features,
+                                go.data_ptr(), None))
+        sync()
+        assert np.array_equal(gf.cpu().numpy().view(np.uint16), feats)
+        assert_close(go.cpu().numpy().view(np.float16).astype(np.float32),
+                     outs.view(np.float16).astype(np.float32), "outputs")
 
 
 # ---- the fused train step -----------------------------------------------------------------
