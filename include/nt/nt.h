@@ -247,8 +247,9 @@ int64_t nt_mip_chain_layout(int width, int height, int num_mips, int64_t *mip_of
 /* The same for 4x4 block storage (blocks per dimension = max(size>>2, 1), train.cu:220). */
 int64_t nt_block_chain_layout(int width, int height, int num_mips, int64_t *block_offset);
 /* Bytes of scratch nt_train_step needs for these parameters (0 on error); also enough for
- * nt_inference's fixed-order SSE. A NT_SAMPLES_RANDOM step of 262,144 samples or more also
- * holds its sample sort (keys, sample indices and per-tile counts, ~12 bytes a sample). */
+ * nt_inference's fixed-order SSE. A NT_SAMPLES_RANDOM step of 262,144 samples or more (65,536
+ * where there is a sample to at most 32 image texels) also holds its sample sort (keys, sample
+ * indices and per-tile counts, ~12 bytes a sample). */
 size_t nt_train_workspace_bytes(const nt_params *params, nt_kernel_type type);
 
 /* Profiling hook (no reference counterpart): the next nt_train_step, nt_optimize_latents,
@@ -264,8 +265,8 @@ int nt_profile_next_launch(void *start_event, void *stop_event);
  *   flags bit 0 (NT_HOOK_DROP_MARGINS) removes the margin of that kernel's chunk cell box,
  *   which drives its latent scatter's out-of-box path (per-sample global atomics);
  *   flags bit 1 (NT_HOOK_SORT_RANDOM) makes NT_SAMPLES_RANDOM steps sort their samples by
- *   bin at any sample count (they do from 262,144 samples), so that small tests reach
- *   the sorted order.
+ *   bin at any sample count (they do from 262,144 samples, or 65,536 where there is one to
+ *   at most 32 image texels), so that small tests reach the sorted order.
  * nt_set_test_hooks(0, 0) restores the defaults. */
 #define NT_HOOK_DROP_MARGINS 1
 #define NT_HOOK_SORT_RANDOM 2
@@ -276,7 +277,7 @@ int nt_set_test_hooks(int max_train_workgroups, int flags);
  * 64 x 64-texel bin (row-major over the image) of their texels (the step then walks each
  * tile of 1,024 of them along a path through its bins). Uses params->workspace
  * (nt_train_workspace_bytes). NT_ERR_UNSUPPORTED when the step trains in slot order
- * (fewer than 262,144 samples without NT_HOOK_SORT_RANDOM, or another kernel). */
+ * (fewer samples than that without NT_HOOK_SORT_RANDOM, or another kernel). */
 int nt_random_sample_order(const nt_params *params, uint32_t *order, void *stream);
 
 /* ---- the hot path ----------------------------------------------------------------- */

@@ -360,11 +360,26 @@ float pow2_reciprocal(int n)
     return n > 0 && (n & (n - 1)) == 0 ? 1.f / (float)n : 0.f;
 }
 
-void plan16(const nt_params *p, nt_kernel_type type, TrainPlan *plan)
+void plan16(const nt_params *p, nt_kernel_type type, TrainPlan *plan, bool bc6_inner_step)
 {
     plan->use16 = 0;
     const bool random = p->sample_mode == NT_SAMPLES_RANDOM;
-    const int NG = train16_groups(plan->shape, random);
+    const int64_t texels = (int64_t)p->image_width * p->image_height;
+    int NG = train16_groups(plan->shape, random);
+    // Random texels run one group of four waves a workgroup instead of two where that puts every
+    // 128 samples on a CU of their own (up to 32,768 on 256 CUs: two grids at 16,384 samples
+    // 39.3 -> 32.2 us, four 153 -> 135), and four grids also where the samples are sparse, at
+    // most one to eight texels: the taps then come from HBM, and the one group, with registers
+    // to issue them at the start of a chunk, waits for them less (four grids, a million samples
+    // of 4096^2 texels: 872 -> 823 us; of 2048^2, one to four texels: 579 -> 619).
+    // (A test hook can lower the workgroups, so that small steps loop and take two groups.)
+    int cap = device_cu_count();
+    if (const int hook = g_hook_max_workgroups.load(std::memory_order_relaxed); hook > 0)
+        cap = std::min(cap, hook);
+    if (random && NG == 2 &&
+        (p->num_samples <= kChunk * cap ||
+         (plan->shape == kShapeC4 && 8 * (int64_t)p->num_samples <= texels)))
+        NG = 1;
     const int C = p->latents.channels, G = p->latents.num_grids;
     // 16-channel grids, or the reference network's four 3-channel grids.
     const bool c3 = plan->shape == kShapeRef;
@@ -427,34 +442,33 @@ void plan16(const nt_params *p, nt_kernel_type type, TrainPlan *plan)
     d.ntex = p->num_textures;
     const int rw = p->region_width > 0 ? p->region_width : NT_DEFAULT_REGION;
     const int rows = (int)(((int64_t)p->num_samples + rw - 1) / rw);
-    // Region: tiles of 16 tile_chunks x 8NG positions. Random texels: tiles of 512 NG consecutive
-    // samples (of the bin order).
+    // Region: tiles of 16 tile_chunks x 8NG positions. Random texels: tiles of 128 tile_chunks NG
+    // consecutive samples (of the bin order).
     // One workgroup per CU (the kernel's registers and LDS allow no second one); each takes
     // every nwg-th tile, so that fewer, longer-lived workgroups stage the weights and write
     // MLP-gradient partials.
-    // A test hook can lower the cap (to give workgroups several tiles at small sizes).
-    int cap = device_cu_count();
-    if (const int hook = g_hook_max_workgroups.load(std::memory_order_relaxed); hook > 0)
-        cap = std::min(cap, hook);
     // A workgroup's time is its chunks in sequence, so a tile has four chunks, or two or one
-    // where that leaves the busiest workgroup fewer of them: whole steps of two grids at 64 x 32
+    // where that leaves the busiest workgroup fewer of them (region and random texels: two grids
+    // at 16,384 random samples 98 -> 32 us): whole region steps of two grids at 64 x 32
     // samples 44.8 -> 21.5 us and at 300 x 217 48.5 -> 32.9 us (one chunk a workgroup, then
     // two); the reference network at 509 x 331, 168 tiles of four on 256 CUs, 76.8 -> 69.2 us
     // (three). Equal counts keep the wider tile (fewer halo texels and box flushes).
-    d.tile_chunks = 4;
-    if (random) {
-        d.tiles_x = 1;
-        const int64_t n = ((int64_t)p->num_samples + 4 * kChunk * NG - 1) / (4 * kChunk * NG);
-        if (n > (1 << 30))
-            return;
-        d.ntiles = (int)n;
-    } else {
+    d.groups = NG;
+    {
         int64_t best = 0;
         for (int tc = 4; tc >= 1; tc /= 2) {
-            const int64_t tx = (rw + tc * kChunkW - 1) / (tc * kChunkW), n = tx * ((rows + kChunkH * NG - 1) / (kChunkH * NG));
-            const int64_t serial = (n + cap - 1) / cap * tc;
+            const int64_t tx = random ? 1 : (rw + tc * kChunkW - 1) / (tc * kChunkW);
+            const int64_t ty = random ? ((int64_t)p->num_samples + tc * kChunk * NG - 1) / (tc * kChunk * NG)
+                                      : (rows + kChunkH * NG - 1) / (kChunkH * NG);
+            const int64_t n = tx * ty, serial = (n + cap - 1) / cap * tc;
             if (n > (1 << 30) || (best > 0 && serial >= best))
                 continue;
+            // A region step with the dense optimizer and fewer than 16 wide tiles keeps them, and
+            // with them its workspace of one gradient row per 64 x 8NG tile, which callers of
+            // such steps size their memory by; an update-log or block-record step's workspace
+            // holds a row per workgroup.
+            if (best > 0 && !random && !bc6_inner_step && p->latent_update == NT_LATENT_DENSE && d.ntiles < 16)
+                break;
             best = serial;
             d.tile_chunks = tc;
             d.tiles_x = (int)tx;
@@ -631,10 +645,15 @@ void plan16(const nt_params *p, nt_kernel_type type, TrainPlan *plan)
     plan->workspace = (size_t)plan->rows * (size_t)plan->P * sizeof(float);
     // Random texels: the sort of the sample indices by bin after the partial rows (keys and
     // sample indices in two buffers each, then the per-tile digit counts). From 262,144
-    // samples: config 2 with random texels runs its train kernel 204 -> 176 us with it,
-    // config 4 (1,048,576 samples) 1,392 -> 1,120 us.
+    // samples (two grids, 2048^2 texels: 231 -> 187 us a step; four, a million of 4096^2: 1,268
+    // -> 823), and from 65,536 where there is a sample to at most 32 texels (four grids, 65,536
+    // of 512^2: 114 -> 84 us; 131,072 of 2048^2: 228 -> 182; sparser, 65,536 of 4096^2: 219,
+    // 241 sorted; fewer, 32,768 of 1024^2: 71, 82 sorted).
     plan->sort_off = plan->sort_temp = 0;
-    if (random && (p->num_samples >= kRandomSortMinSamples || g_hook_sort_random.load(std::memory_order_relaxed))) {
+    const bool sorted = p->num_samples >= kRandomSortMinSamples ||
+                        (p->num_samples >= kRandomSortMinDense && 32 * (int64_t)p->num_samples >= texels) ||
+                        g_hook_sort_random.load(std::memory_order_relaxed);
+    if (random && sorted) {
         // Bins of 64 x 64 texels (coarser ones, one 8-bit sort pass, gained less).
         const int shift = 6;
         const int bx = (p->image_width + (1 << shift) - 1) >> shift;
@@ -706,7 +725,7 @@ nt_params bc6_inner(const nt_params *p, const TrainPlan &plan, uint8_t *ws)
     return q;
 }
 
-int plan_train(const nt_params *p, nt_kernel_type type, TrainPlan *plan);
+int plan_train(const nt_params *p, nt_kernel_type type, TrainPlan *plan, bool bc6_inner_step = false);
 
 // The BC6 block phase (NT_BLOCK_FEATURES, NT_FINALIZE) runs an unconstrained train step on
 // texels expanded from the block records of every level a sample reaches (Bc6PhaseDesc):
@@ -736,7 +755,7 @@ void plan_bc6_phase(const nt_params *p, TrainPlan *plan)
     }
     const nt_params q = bc6_inner(p, t, nullptr);
     TrainPlan inner;
-    if (plan_train(&q, NT_UNCONSTRAINED, &inner) != NT_OK)
+    if (plan_train(&q, NT_UNCONSTRAINED, &inner, true) != NT_OK)
         return;
     // The inner plan, with the phase's fields.
     for (int gi = 0; gi < G; ++gi)
@@ -791,7 +810,7 @@ void plan_bc6_phase(const nt_params *p, TrainPlan *plan)
     *plan = inner;
 }
 
-int plan_train(const nt_params *p, nt_kernel_type type, TrainPlan *plan)
+int plan_train(const nt_params *p, nt_kernel_type type, TrainPlan *plan, bool bc6_inner_step)
 {
     if (!p)
         return fail(NT_ERR_NULL_POINTER, "params is NULL");
@@ -919,7 +938,7 @@ int plan_train(const nt_params *p, nt_kernel_type type, TrainPlan *plan)
     }
     plan->rows = plan->nwg;
     plan->bc6 = 0;
-    plan16(p, type, plan);
+    plan16(p, type, plan, bc6_inner_step);
     if (type != NT_UNCONSTRAINED)
         plan_bc6_phase(p, plan);
     if (type != NT_UNCONSTRAINED && !plan->bc6)
@@ -1344,8 +1363,9 @@ int nt_random_sample_order(const nt_params *p, uint32_t *order, void *stream)
         return fail(NT_ERR_NULL_POINTER, "order");
     if (!plan.use16 || !plan.sort_off)
         return fail(NT_ERR_UNSUPPORTED, "these parameters train in slot order (the sort: NT_SAMPLES_RANDOM on the "
-                                        "16-channel kernel, from %d samples or with NT_HOOK_SORT_RANDOM)",
-                    kRandomSortMinSamples);
+                                        "16-channel kernel, from %d samples, %d where there is one to at most 32 texels, "
+                                        "or with NT_HOOK_SORT_RANDOM)",
+                    kRandomSortMinSamples, kRandomSortMinDense);
     if (!p->workspace || p->workspace_bytes < plan.workspace)
         return fail(NT_ERR_WORKSPACE, "workspace of %zu bytes needed, %zu given", plan.workspace,
                     p->workspace ? p->workspace_bytes : (size_t)0);

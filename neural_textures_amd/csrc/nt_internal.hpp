@@ -123,7 +123,8 @@ struct Grid16 {
 // NT_SAMPLES_RANDOM: the sample indices sorted by the 64 x 64-texel bin of their texels
 // (nt_sort.hip). Keys and sample indices in two buffers each (the counting sort's two passes)
 // and the per-tile digit counts, all in the train workspace.
-constexpr int kRandomSortMinSamples = 1 << 18; // fewer samples train in slot order
+constexpr int kRandomSortMinSamples = 1 << 18; // fewer samples train in slot order ...
+constexpr int kRandomSortMinDense = 1 << 16;   // ... or, with one to at most 32 texels, fewer than these
 constexpr int kRandomSortTile = 4096;          // samples per workgroup in the counting passes
 constexpr int kRandomSortMaxTiles = 256;       // more samples make the tiles longer
 struct RandomOrderDesc {
@@ -174,7 +175,8 @@ struct Train16Desc {
     // 1/image_w, 1/image_h, 1/num_samples where that is a power of two (a product with the
     // reciprocal then equals the quotient exactly), else 0 (divide).
     float inv_w, inv_h, inv_samples;
-    int tile_chunks; // region: 16-position chunks across a tile (1, 2 or 4)
+    int groups;      // groups of four waves a workgroup (the kernel's NG)
+    int tile_chunks; // chunks a tile, one after another (1, 2 or 4); region: side by side
     int tiles_x, ntiles, nwg, xcd_per; // xcd_per > 0: workgroups of one XCD take consecutive tiles
     int group_off, group_bytes, tile_bytes; // per 4-wave group: target tile, then the union
     int wcols;                              // halves per scatter-weight row (one row per sample)
@@ -188,8 +190,8 @@ struct Train16Desc {
     // reads global memory.
     int gbox_off, gbox_bytes, gbox_items;
     // NT_SAMPLES_RANDOM: positions at uniformly random texels of the image; no target tile
-    // (taps read from global memory) and per-sample gradient atomics instead of the
-    // chunk-box reduction; tiles of 512 consecutive samples.
+    // (taps read from global memory); in slot order per-sample gradient atomics, in bin order
+    // each wave's cell-box reduction; tiles of 128 tile_chunks groups consecutive samples.
     int random_texels;
     const uint32_t *order; // random texels: the sample of each slot (NULL: slot i is sample i)
     uint64_t perm;                          // nibble r: output index of output row r

@@ -1330,7 +1330,7 @@ __global__ __launch_bounds__(kTrainThreads *NG) void train16_kernel(Train16Desc 
         }
     }
 
-    const int nchunk = NARROW ? d.tile_chunks : 4;
+    const int nchunk = NARROW || RND ? d.tile_chunks : 4;
     for (int chunk = 0; chunk < nchunk; ++chunk) {
         const int cx0 = d.off_x + tx0 + chunk * kChunkW, cy0 = d.off_y + ty0 + kChunkH * gr;
         // With gather boxes both copies are untracked: the gather's LDS reads (another buffer)
@@ -1347,9 +1347,10 @@ __global__ __launch_bounds__(kTrainThreads *NG) void train16_kernel(Train16Desc 
         uint32_t sidx = (uint32_t)sy * (uint32_t)d.region_w + (uint32_t)sx;
         bool valid = sx < d.region_w && sidx < (uint32_t)d.num_samples;
         if constexpr (RND) {
-            // Slot 512 (NG b + gr) + 128 chunk + 32 wave + c: tiles of consecutive slots; with
+            // Slot 128 ((NG b + gr) nchunk + chunk) + 32 wave + c: tiles of consecutive slots; with
             // ORD each holds the sample the bin-sorted order gives it, else slot i is sample i.
-            sidx = (((((uint32_t)b * NG + (uint32_t)gr) * 4u + (uint32_t)chunk) * 4u + (uint32_t)wave) * 32u) +
+            sidx = (((((uint32_t)b * NG + (uint32_t)gr) * (uint32_t)nchunk + (uint32_t)chunk) * 4u + (uint32_t)wave) *
+                    32u) +
                    (uint32_t)c;
             valid = sidx < (uint32_t)d.num_samples;
             if constexpr (ORD) {
@@ -1957,19 +1958,26 @@ static hipError_t launch16(const Train16Desc &d, size_t lds, hipStream_t s)
 }
 
 // This file is compiled twice: once for the region kernels and the host functions below,
-// and once with NT_TRAIN16_RANDOM_UNIT for the random-texel kernels alone, under the
+// and once with NT_TRAIN16_RANDOM_UNIT for the random-texel kernels alone (one and two
+// groups), under the
 // scheduler that groups memory instructions into clauses
 // (-amdgpu-sched-strategy=max-memory-clause): the random-texel kernels wait on their
 // gathers, taps and atomics, and that schedule runs the config-2 one 4 % faster (214 -> 205
 // us in alternating runs) while the region kernels run as fast or slower with it.
 #ifdef NT_TRAIN16_RANDOM_UNIT
+template <class S, int NG>
+static hipError_t launch_random(const Train16Desc &d, size_t lds, hipStream_t s)
+{
+    return d.order ? launch16<S, 16, NG, true, true>(d, lds, s) : launch16<S, 16, NG, true>(d, lds, s);
+}
+
 hipError_t launch_train16_random(int shape, const Train16Desc &d, size_t lds, hipStream_t s)
 {
     switch (shape) {
     case kShapeC2:
-        return d.order ? launch16<ShapeC2, 16, 2, true, true>(d, lds, s) : launch16<ShapeC2, 16, 2, true>(d, lds, s);
+        return d.groups == 1 ? launch_random<ShapeC2, 1>(d, lds, s) : launch_random<ShapeC2, 2>(d, lds, s);
     case kShapeC4:
-        return d.order ? launch16<ShapeC4, 16, 2, true, true>(d, lds, s) : launch16<ShapeC4, 16, 2, true>(d, lds, s);
+        return d.groups == 1 ? launch_random<ShapeC4, 1>(d, lds, s) : launch_random<ShapeC4, 2>(d, lds, s);
     default:
         return hipErrorInvalidValue;
     }

@@ -313,10 +313,17 @@ def test_train_step_tile_widths(lib, O, shape, rows, max_wg, ragged):
     one row shorter) over one, three, four and enough workgroups: tiles of four, two and one
     chunks, the one that leaves the busiest workgroup the fewest. Gradients match the oracle's."""
     say(f"case: tile widths {shape} workgroups {max_wg} ragged {ragged}")
+    st = make_state(shape, image=256, region=(128 - ragged, rows - (ragged > 0)), seed=3,
+                    offset=(21, 240 if ragged else 7))
+    st.latent_update = abi.NT_LATENT_TOUCHED  # (a small dense step keeps wide tiles)
+    alt, gs = st.converted(False), st.to_torch()
+    oracle_step(O, st, 0)
+    oracle_step(O, alt, 0, accum_f32=True)
     nt.check(lib.nt_set_test_hooks(max_wg, 0))
     try:
-        st, gs, alt = run_train_pair(lib, O, shape, 256, (128 - ragged, rows - (ragged > 0)), (21, 240 if ragged else 7),
-                                     abi.NT_UNCONSTRAINED, seed=3)
+        gs = gpu_workspace(lib, gs, 0)
+        nt.check(lib.nt_train_step(C.byref(gs.params()), 0, None))
+        sync()
     finally:
         nt.check(lib.nt_set_test_hooks(0, 0))
     check_train_grads(st, gs, alt)
@@ -394,6 +401,23 @@ def test_random_texel_path_scatter(lib, O, shape, image, n, overflow):
         assert np.array_equal(np.isfinite(got), np.isfinite(h.grads))
         fine = np.isfinite(got)
         assert_close(got[fine], h.grads[fine], "finite latent gradients")
+
+
+@pytest.mark.parametrize("shape", ["c2", "c4"])
+@pytest.mark.parametrize("image,n,max_wg", [(64, 127, 0), (64, 129, 1), (64, 640, 2), (64, 1300, 2), (512, 1300, 2),
+                                            (64, 2100, 3)])
+def test_train_step_random_tiles(lib, O, shape, image, n, max_wg):
+    """NT_SAMPLES_RANDOM tiles of one, two and four chunks in one and two groups (n samples on at
+    most max_wg workgroups; four sparse grids take one group), the last partial: gradients match
+    the oracle's."""
+    say(f"case: random tiles {shape} image {image} samples {n} workgroups {max_wg}")
+    nt.check(lib.nt_set_test_hooks(max_wg, 0))
+    try:
+        st, gs, alt = run_train_pair(lib, O, shape, image, (n, 1), (0, 0), abi.NT_UNCONSTRAINED, seed=19,
+                                     sample_mode=abi.NT_SAMPLES_RANDOM)
+    finally:
+        nt.check(lib.nt_set_test_hooks(0, 0))
+    check_train_grads(st, gs, alt)
 
 
 def test_random_texel_sorted_step_is_deterministic(lib):
