@@ -802,7 +802,7 @@ void plan_bc6_phase(const nt_params *p, TrainPlan *plan)
             x.nby = x.nbv;
         }
         x.first_block = first;
-        first += (int64_t)x.nbx * x.nby;
+        first += ((int64_t)x.nbx * x.nby + kBc6PhaseBlocks - 1) / kBc6PhaseBlocks * kBc6PhaseBlocks;
     }
     b.total_blocks = first;
     inner.workspace = off;

@@ -235,15 +235,31 @@ hipError_t launch_bc6_init(const Bc6InitDesc &d, hipStream_t s)
 
 // ---- the BC6 block phase on the fused train kernel ------------------------------------
 
-// The level of a launch-wide block number (levels take consecutive ranges of blocks).
-__device__ __forceinline__ int bc6_phase_level(const Bc6PhaseDesc &d, int64_t b)
+// The level of the workgroup (16 blocks, all of one level: levels start at multiples of
+// kBc6PhaseBlocks): uniform, so that its fields are scalar loads.
+__device__ __forceinline__ int bc6_phase_level(const Bc6PhaseDesc &d)
 {
+    const int b = (int)blockIdx.x * kBc6PhaseBlocks;
     int li = 0;
 #pragma unroll
     for (int k = 1; k < 2 * NT_MAX_GRIDS; ++k)
         if (k < d.nlevels && b >= d.level[k].first_block)
             li = k;
-    return li;
+    return __builtin_amdgcn_readfirstlane(li);
+}
+
+// The 32 partition masks in LDS: a table indexed by a loaded value is otherwise a memory load
+// that waits for that value. The caller synchronises before using it.
+__device__ __forceinline__ void bc6_stage_masks(int *masks)
+{
+    if (threadIdx.x < 32)
+        masks[threadIdx.x] = bc6_partition_mask((int)threadIdx.x);
+}
+// bc6_mode_bits without its table: four bits a mode.
+__device__ __forceinline__ int bc6_mode_bits_packed(int m)
+{
+    constexpr uint64_t kBits = 0x6888'9BBB'7Aull; // modes 9 .. 0: 6 8 8 8 9 11 11 11 7 10
+    return (int)(kBits >> (4 * ((unsigned)m < 10u ? (unsigned)m : 0u))) & 15;
 }
 
 __device__ __forceinline__ int wrap_mod(int v, int n)
@@ -281,29 +297,41 @@ __device__ __forceinline__ void bc6_block_of(const Bc6PhaseLevel &g, int lb, int
 // picks the endpoints afterwards): the four endpoints of every channel, the pixel's index
 // on the segment, the partition and the mode.
 template <int C>
+struct Bc6Raw {
+    float e[4][C], xi;
+    int partition, mode;
+};
+template <int C>
+__device__ __forceinline__ Bc6Raw<C> bc6_load(const float *rec, int pix)
+{
+    Bc6Raw<C> r;
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+#pragma unroll
+        for (int ch = 0; ch < C; ++ch)
+            r.e[k][ch] = load_global(rec + k * C + ch);
+    r.xi = load_global(rec + 4 * C + pix);
+    r.partition = __float_as_int(load_global(rec + 4 * C + 16));
+    r.mode = __float_as_int(load_global(rec + 4 * C + 17));
+    return r;
+}
+template <int C>
 struct Bc6Pixel {
     float q0[C], q1[C]; // the pixel's partition's endpoints, unquantized
     float xi;
     int part, bits;
 };
 template <int C>
-__device__ __forceinline__ Bc6Pixel<C> bc6_pixel(const float *rec, int pix)
+__device__ __forceinline__ Bc6Pixel<C> bc6_pixel(const Bc6Raw<C> &r, const int *masks, int pix)
 {
-    float e[4][C];
-#pragma unroll
-    for (int k = 0; k < 4; ++k)
-#pragma unroll
-        for (int ch = 0; ch < C; ++ch)
-            e[k][ch] = rec[k * C + ch];
     Bc6Pixel<C> q;
-    q.xi = rec[4 * C + pix];
-    const int partition = __float_as_int(rec[4 * C + 16]);
-    q.bits = bc6_mode_bits(__float_as_int(rec[4 * C + 17]));
-    q.part = (bc6_partition_mask(partition) >> pix) & 1;
+    q.xi = r.xi;
+    q.bits = bc6_mode_bits_packed(r.mode);
+    q.part = (masks[r.partition & 31] >> pix) & 1;
 #pragma unroll
     for (int ch = 0; ch < C; ++ch) {
-        q.q0[ch] = bc6_unquantize(q.part ? e[2][ch] : e[0][ch], q.bits);
-        q.q1[ch] = bc6_unquantize(q.part ? e[3][ch] : e[1][ch], q.bits);
+        q.q0[ch] = bc6_unquantize(q.part ? r.e[2][ch] : r.e[0][ch], q.bits);
+        q.q1[ch] = bc6_unquantize(q.part ? r.e[3][ch] : r.e[1][ch], q.bits);
     }
     return q;
 }
@@ -315,20 +343,20 @@ __device__ __forceinline__ Bc6Pixel<C> bc6_pixel(const float *rec, int pix)
 template <int C>
 __global__ __launch_bounds__(256) void bc6_expand_kernel(Bc6PhaseDesc d)
 {
-    const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    const int64_t b = t >> 4;
-    if (b >= d.total_blocks)
-        return;
-    const Bc6PhaseLevel &g = d.level[bc6_phase_level(d, b)];
-    // A level's rectangle holds fewer than 2^31 blocks (its texels fit 32-bit offsets).
-    const int lb = (int)(b - g.first_block);
-    int bx, by;
-    bc6_block_of(g, lb, bx, by);
-    const int pix = (int)(t & 15);
+    __shared__ int masks[32];
+    const Bc6PhaseLevel &g = d.level[bc6_phase_level(d)];
+    const int lb = (int)(blockIdx.x * kBc6PhaseBlocks - g.first_block) + (int)(threadIdx.x >> 4);
+    const int pix = (int)(threadIdx.x & 15);
+    const bool on = lb < g.nbx * g.nby; // the level's last workgroup may have fewer blocks
+    int bx = 0, by = 0;
+    bc6_block_of(g, on ? lb : 0, bx, by);
+    const Bc6Raw<C> r = bc6_load<C>(g.params + ((int64_t)by * g.nbu + bx) * (4 * C + 18), pix);
+    bc6_stage_masks(masks);
+    __syncthreads();
     const int x = 4 * bx + (pix & 3), y = 4 * by + (pix >> 2);
-    if (x >= g.w || y >= g.h)
+    if (!on || x >= g.w || y >= g.h)
         return; // a level narrower than a block (w or h < 4)
-    const Bc6Pixel<C> q = bc6_pixel<C>(g.params + ((int64_t)by * g.nbu + bx) * (4 * C + 18), pix);
+    const Bc6Pixel<C> q = bc6_pixel<C>(r, masks, pix);
     const int64_t o = ((int64_t)y * g.w + x) * C;
 #pragma unroll
     for (int ch = 0; ch < C; ++ch) {
@@ -350,9 +378,9 @@ __global__ __launch_bounds__(256) void bc6_expand_kernel(Bc6PhaseDesc d)
 // exact, so the sums over corners equal these terms applied to the texel's gradient
 // G = sum w g (which the fused kernel accumulated) up to the order of the fp32 additions
 // (which the reference's atomics leave open as well). The pixel thread adds its pixel-index
-// gradient; the endpoint terms are summed over the block's 16 threads with lane shuffles
-// and added by its first thread. Texels with a zero gradient add nothing; each record field
-// is read, added to and written by one thread only.
+// gradient; the endpoint terms are summed over the block's 16 threads with lane shuffles and
+// each added by one of them. Texels with a zero gradient add nothing; each record field is
+// read, added to and written by one thread only.
 template <int C>
 __global__ __launch_bounds__(256) void bc6_fold_kernel(Bc6PhaseDesc d)
 {
@@ -375,37 +403,46 @@ __global__ __launch_bounds__(256) void bc6_fold_kernel(Bc6PhaseDesc d)
                     log->rect[gi][k] = d.rect[gi][k];
         }
     }
-    // The 16 threads of a block are 16 consecutive lanes of one wave (the launch covers
-    // whole blocks), so every cross-lane sum below stays within the block's lanes, and
-    // a block's lanes leave only together.
-    const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    const int64_t b = t >> 4;
-    if (b >= d.total_blocks)
-        return;
-    const Bc6PhaseLevel &g = d.level[bc6_phase_level(d, b)];
-    // A level's rectangle holds fewer than 2^31 blocks (its texels fit 32-bit offsets).
-    const int lb = (int)(b - g.first_block);
-    int bx, by;
-    bc6_block_of(g, lb, bx, by);
-    const int pix = (int)(t & 15);
+    // The 16 threads of a block are 16 consecutive lanes of one wave, so every cross-lane sum
+    // below stays within the block's lanes, and a block's lanes leave only together. The
+    // record, the texel gradients and the record gradients it adds to are all loaded at once
+    // (nearly every block of the rectangle is touched); lane p adds the pixel-index gradient p
+    // and the endpoint gradients p, p + 16, ... of the record.
+    __shared__ int masks[32];
+    const Bc6PhaseLevel &g = d.level[bc6_phase_level(d)];
+    const int lb = (int)(blockIdx.x * kBc6PhaseBlocks - g.first_block) + (int)(threadIdx.x >> 4);
+    const int pix = (int)(threadIdx.x & 15);
+    const bool on = lb < g.nbx * g.nby;
+    int bx = 0, by = 0;
+    bc6_block_of(g, on ? lb : 0, bx, by);
     const int64_t blk = (int64_t)by * g.nbu + bx;
     const int x = 4 * bx + (pix & 3), y = 4 * by + (pix >> 2);
-    const bool inside = x < g.w && y < g.h; // a level narrower than a block (w or h < 4)
+    const bool inside = on && x < g.w && y < g.h; // a level narrower than a block (w or h < 4)
     const int64_t o = ((int64_t)y * g.w + x) * C;
     float G[C];
+#pragma unroll
+    for (int ch = 0; ch < C; ++ch)
+        G[ch] = inside ? load_global(g.tgrads + o + ch) : 0.f;
+    const Bc6Raw<C> raw = bc6_load<C>(g.params + blk * (4 * C + 18), pix);
+    constexpr int NE = (4 * C + 15) / 16; // endpoint gradients a lane
+    float *grec = g.grads + blk * (4 * C + 16);
+    const float old_pix = load_global(grec + 4 * C + pix);
+    float old_end[NE];
+#pragma unroll
+    for (int i = 0; i < NE; ++i)
+        old_end[i] = load_global(grec + min(pix + 16 * i, 4 * C - 1));
+    bc6_stage_masks(masks);
+    __syncthreads();
     bool touched = false;
 #pragma unroll
-    for (int ch = 0; ch < C; ++ch) {
-        G[ch] = inside ? g.tgrads[o + ch] : 0.f;
+    for (int ch = 0; ch < C; ++ch)
         touched |= G[ch] != 0.f;
-    }
     // Lanes of the block with a non-zero gradient (the block's 16-bit slice of the wave's).
     const uint64_t vote = __ballot(touched);
     const int lane = (int)(threadIdx.x & 63);
     if (((vote >> (lane & ~15)) & 0xFFFFull) == 0)
         return; // the whole block untouched (all 16 lanes leave together)
-    const Bc6Pixel<C> q = bc6_pixel<C>(g.params + blk * (4 * C + 18), pix);
-    float *grec = g.grads + blk * (4 * C + 16);
+    const Bc6Pixel<C> q = bc6_pixel<C>(raw, masks, pix);
     const float deibar = ldexpf(31.f / 64.f, 16 - q.bits);
     const float alpha = ldexpf(q.xi, 3);
     float dl_dx = 0.f;
@@ -423,11 +460,15 @@ __global__ __launch_bounds__(256) void bc6_fold_kernel(Bc6PhaseDesc d)
         de[3][ch] = q.part ? a1 : 0.f;
     }
     if (touched)
-        grec[4 * C + pix] += dl_dx;
+        grec[4 * C + pix] = old_pix + dl_dx;
     // Sums over the block's 16 lanes by DPP within each row of 16: lanes xor 1, xor 2
     // (quad permutations), then the mirrors of each half row and of the row (after the
     // first two steps every lane of a quad holds the quad's sum, and each mirror pairs every
-    // lane with one of the other half).
+    // lane with one of the other half). Every lane ends with every sum.
+    float mine[NE];
+#pragma unroll
+    for (int i = 0; i < NE; ++i)
+        mine[i] = 0.f;
 #pragma unroll
     for (int k = 0; k < 4; ++k)
 #pragma unroll
@@ -437,16 +478,13 @@ __global__ __launch_bounds__(256) void bc6_fold_kernel(Bc6PhaseDesc d)
             v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x4E, 0xF, 0xF, false));
             v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x141, 0xF, 0xF, false));
             v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x140, 0xF, 0xF, false));
-            de[k][ch] = v;
+            const int e = k * C + ch;
+            mine[e / 16] = pix == e % 16 ? v : mine[e / 16];
         }
-    if (pix == 0) {
 #pragma unroll
-        for (int k = 0; k < 4; ++k)
-#pragma unroll
-            for (int ch = 0; ch < C; ++ch)
-                if (de[k][ch] != 0.f)
-                    grec[k * C + ch] += de[k][ch];
-    }
+    for (int i = 0; i < NE; ++i)
+        if (pix + 16 * i < 4 * C && mine[i] != 0.f)
+            grec[pix + 16 * i] = old_end[i] + mine[i];
 }
 
 template <template <int> class K>
@@ -454,7 +492,7 @@ static hipError_t launch_phase(const Bc6PhaseDesc &d, hipStream_t s)
 {
     if (d.total_blocks <= 0)
         return hipSuccess;
-    const dim3 grid((unsigned)((d.total_blocks * 16 + 255) / 256));
+    const dim3 grid((unsigned)(d.total_blocks / kBc6PhaseBlocks));
     switch (d.C) {
     case 3:
         hipLaunchKernelGGL(K<3>::kernel, grid, dim3(256), 0, s, d);

@@ -296,10 +296,11 @@ struct Bc6PhaseLevel {
     int bx0, by0, nbx, nby; // block rectangle: origin (may lie outside the level: wraps), size
     int64_t first_block;    // first block of this level in the launch's numbering
 };
+constexpr int kBc6PhaseBlocks = 16; // blocks a workgroup; levels start at multiples of it
 struct Bc6PhaseDesc {
     Bc6PhaseLevel level[2 * NT_MAX_GRIDS];
     int nlevels, C;
-    int64_t total_blocks;
+    int64_t total_blocks; // the levels' blocks, each rounded up to whole workgroups
     // NT_LATENT_TOUCHED with one level per grid (mip 0): the update log, in which the fold
     // records each grid's block rectangle {bx0, bx1, by0, by1} (inclusive, before wrapping);
     // NULL: none.
