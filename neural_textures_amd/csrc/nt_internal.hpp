@@ -175,8 +175,6 @@ struct Train16Desc {
     // 1/image_w, 1/image_h, 1/num_samples where that is a power of two (a product with the
     // reciprocal then equals the quotient exactly), else 0 (divide).
     float inv_w, inv_h, inv_samples;
-    int groups;      // groups of four waves a workgroup (the kernel's NG)
-    int tile_chunks; // chunks a tile, one after another (1, 2 or 4); region: side by side
     int tiles_x, ntiles, nwg, xcd_per; // xcd_per > 0: workgroups of one XCD take consecutive tiles
     int group_off, group_bytes, tile_bytes; // per 4-wave group: target tile, then the union
     int wcols;                              // halves per scatter-weight row (one row per sample)
@@ -202,6 +200,8 @@ struct Train16Desc {
     // corner of the region's positions.
     struct UpdateLog *log;
     int32_t rect[NT_MAX_GRIDS][4];
+    int groups;      // groups of four waves a workgroup (the kernel's NG)
+    int tile_chunks; // chunks a tile, one after another (1, 2 or 4); region: side by side
 };
 
 // NT_LATENT_TOUCHED: the update log, the last kUpdateLogBytes of the train workspace. A
