@@ -13,12 +13,18 @@
 // LDS (the whole key when it has at most ten bits, config 2's 1,024 bins; else its top eight
 // bits). sort_first_pass_kernel: each workgroup derives where its tile's samples of each
 // digit start from all tiles' counts (the digits' totals, scanned, plus the digit's counts
-// in earlier tiles), then places its samples in order, 256 a round (the keys of 16 rounds
-// loaded at once, so that the rounds wait on no memory): a sample's place is its digit's
-// running place + the samples before it in the round with the same digit (a wave's lanes by
-// ballots on the digit bits, the waves before it by their counts). Keys of more than ten
+// in earlier tiles). Each of its eight waves then places a contiguous part of the tile in
+// order, 64 a round: it has its own row of running places (the tile's, plus the counts of the
+// waves before it), so a sample's place is its digit's entry + the lanes before it with the
+// same digit (ballots on the digit bits), and rounds need no barrier. Keys of more than ten
 // bits then go through sort_segment_kernel: one workgroup per first digit sorts that digit's
 // segment by the remaining key bits the same way, writing the final order.
+//
+// What bounds it: the latency of the rounds. With one row of places a workgroup of 256 and
+// two barriers in each round of 256 items, the first pass took 19.3 us for 262,144 samples in
+// 1,024 bins (64 workgroups), now 12.1; for a million samples in 4,096 bins 20.3 -> 18.1 us (the
+// scattered stores of two arrays) and the segments 13.3 -> 9.7 us. A step of two grids 188.7 ->
+// 180.5 us, of four 823 -> 814 us. More threads in the count kernel (1,024) gain nothing.
 #include <hip/hip_runtime.h>
 
 #include "nt_internal.hpp"
@@ -27,8 +33,9 @@ namespace ntk {
 
 namespace {
 
-constexpr int kSortThreads = 256, kSortWaves = kSortThreads / 64;
-constexpr int kSortRegs = 16;   // items per thread loaded at once in the scatter passes
+constexpr int kSortThreads = 256; // the counts and the path
+constexpr int kPassThreads = 512, kPassWaves = kPassThreads / 64;
+constexpr int kPassRegs = 8; // items per lane loaded at once: a wave's part of a tile of 4,096
 constexpr int kSortMaxDigits = 1024; // digits of a one-pass sort (keys of at most ten bits)
 
 __device__ __forceinline__ uint32_t bin_key(const RandomOrderDesc &d, uint32_t i)
@@ -50,38 +57,61 @@ __device__ __forceinline__ uint64_t match_digit(uint32_t digit, int bits, uint64
     return m;
 }
 
-// One round of a stable counting-sort pass over 256 items (item t of the round on thread t).
-// base[x]: where the next item of digit x goes; wcnt[w][x]: wave w's count of digit x in the
-// round, zero outside the round (each wave writes and clears only its own row). The first
-// barrier also orders the previous round's additions to base before this round reads it.
-// Returns the item's place (valid items only).
-template <int ND>
-__device__ __forceinline__ uint32_t round_place(uint32_t digit, int bits, bool valid, uint32_t *base,
-                                                uint32_t (*wcnt)[ND])
+// Writes to a wave's own LDS row are read by other lanes of the same wave: no barrier.
+__device__ __forceinline__ void wave_order()
 {
-    const int t = threadIdx.x, w = t >> 6, lane = t & 63;
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// One round of a wave's stable counting-sort pass over 64 items, one a lane. row[x]: where the
+// wave's next item of digit x goes. Returns the item's place (valid items only).
+__device__ __forceinline__ uint32_t round_place(uint32_t digit, int bits, bool valid, uint32_t *row)
+{
     const uint64_t m = match_digit(digit, bits, __ballot(valid));
-    const uint64_t before = m & ((1ull << lane) - 1ull);
-    const bool leader = valid && before == 0; // the lowest lane of each digit
-    const uint32_t cnt = (uint32_t)__popcll(m);
-    if (leader)
-        wcnt[w][digit] = cnt;
-    __syncthreads();
-    uint32_t pos = 0;
-    if (valid) {
-        pos = base[digit] + (uint32_t)__popcll(before);
+    const uint64_t before = m & ((1ull << (threadIdx.x & 63)) - 1ull);
+    const uint32_t place = valid ? row[digit] : 0u;
+    wave_order();
+    if (valid && before == 0) // the lowest lane of each digit
+        row[digit] = place + (uint32_t)__popcll(m);
+    wave_order();
+    return place + (uint32_t)__popcll(before);
+}
+
+// The sum of s over the threads before this one (part: a word per wave).
+__device__ __forceinline__ uint32_t exclusive_scan(uint32_t s, uint32_t *part)
+{
+    const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+    uint32_t inc = s;
 #pragma unroll
-        for (int v = 0; v < kSortWaves - 1; ++v) {
-            const uint32_t x = wcnt[v][digit];
-            pos += v < w ? x : 0u;
-        }
+    for (int off = 1; off < 64; off <<= 1) {
+        const uint32_t x = __shfl_up(inc, off);
+        inc += lane >= off ? x : 0u;
     }
+    if (lane == 63)
+        part[w] = inc;
     __syncthreads();
-    if (leader) {
-        atomicAdd(&base[digit], cnt); // integer adds: the same sum in any order
-        wcnt[w][digit] = 0;
+    uint32_t run = inc - s;
+#pragma unroll
+    for (int v = 0; v < kPassWaves - 1; ++v)
+        run += v < w ? part[v] : 0u;
+    return run;
+}
+
+// A digit's counts of every wave, turned into the waves' first places from `run` on.
+template <int ND>
+__device__ __forceinline__ void wave_places(uint32_t (*rows)[ND], int digit, uint32_t run)
+{
+    uint32_t c[kPassWaves];
+#pragma unroll
+    for (int v = 0; v < kPassWaves; ++v)
+        c[v] = rows[v][digit];
+#pragma unroll
+    for (int v = 0; v < kPassWaves; ++v) {
+        rows[v][digit] = run;
+        run += c[v];
     }
-    return pos;
 }
 
 // Counts per tile and first digit: tile-major rows of max(4, digits) counts.
@@ -110,14 +140,14 @@ __global__ __launch_bounds__(kSortThreads) void sort_count_kernel(RandomOrderDes
 
 // base[x] (x < max(4, digits)): where this workgroup's first sample of first digit x goes.
 // Thread t sums digits 4g .. 4g + 3 (g = t mod G, G = max(4, digits) / 4 groups) over the
-// tiles of range t / G (256 / G ranges), 16-byte loads issued 16 at a time; the ranges are
+// tiles of range t / G (512 / G ranges), 16-byte loads issued 16 at a time; the ranges are
 // added in LDS, then the groups' totals scanned.
-__device__ __forceinline__ void tile_bases(const RandomOrderDesc &d, uint32_t *base, uint32_t (*red)[kSortThreads][4],
+__device__ __forceinline__ void tile_bases(const RandomOrderDesc &d, uint32_t *base, uint32_t (*red)[kPassThreads][4],
                                            uint32_t *part)
 {
     const int t = threadIdx.x, tile = blockIdx.x;
     const int ndig = 1 << d.high_bits, stride = ndig < 4 ? 4 : ndig;
-    const int groups = stride / 4, ranges = kSortThreads / groups;
+    const int groups = stride / 4, ranges = kPassThreads / groups;
     const int g = t % groups, r = t / groups;
     const int per = (d.tiles + ranges - 1) / ranges, b_lo = min(r * per, d.tiles), b_hi = min(b_lo + per, d.tiles);
     uint32_t tot[4] = {0u, 0u, 0u, 0u}, pre[4] = {0u, 0u, 0u, 0u};
@@ -155,16 +185,8 @@ __device__ __forceinline__ void tile_bases(const RandomOrderDesc &d, uint32_t *b
             }
         s = tot[0] + tot[1] + tot[2] + tot[3];
     }
-    part[t] = s;
-    __syncthreads();
-    for (int off = 1; off < kSortThreads; off <<= 1) {
-        const uint32_t x = t >= off ? part[t - off] : 0u;
-        __syncthreads();
-        part[t] += x;
-        __syncthreads();
-    }
+    uint32_t run = exclusive_scan(s, part);
     if (t < groups) {
-        uint32_t run = part[t] - s;
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
             base[4 * t + c] = run + pre[c];
@@ -177,40 +199,58 @@ __device__ __forceinline__ void tile_bases(const RandomOrderDesc &d, uint32_t *b
 // The first pass (see the top of the file): the final order for keys of at most ten bits;
 // else keys and sample indices into the alternate buffers, grouped by their top eight bits,
 // and (workgroup 0) each group's start.
-__global__ __launch_bounds__(kSortThreads) void sort_first_pass_kernel(RandomOrderDesc d)
+__global__ __launch_bounds__(kPassThreads) void sort_first_pass_kernel(RandomOrderDesc d)
 {
     __shared__ uint32_t base[kSortMaxDigits];
-    __shared__ uint32_t wcnt[kSortWaves][kSortMaxDigits];
-    __shared__ uint32_t red[2][kSortThreads][4];
-    __shared__ uint32_t part[kSortThreads];
-    const int t = threadIdx.x;
+    __shared__ uint32_t rows[kPassWaves][kSortMaxDigits];
+    __shared__ uint32_t red[2][kPassThreads][4];
+    __shared__ uint32_t part[kPassWaves];
+    const int t = threadIdx.x, lane = t & 63, w = __builtin_amdgcn_readfirstlane(t >> 6);
     const int ndig = 1 << d.high_bits, low = d.key_bits - d.high_bits;
-    for (int v = 0; v < kSortWaves; ++v)
-        for (int x = t; x < kSortMaxDigits; x += kSortThreads)
-            wcnt[v][x] = 0;
+    for (int x = t; x < kPassWaves * kSortMaxDigits; x += kPassThreads)
+        rows[0][x] = 0;
+    __syncthreads();
+    // The wave's part of the tile.
+    const int64_t end = min((int64_t)(blockIdx.x + 1) * d.tile, (int64_t)d.n);
+    const int per = (d.tile + kPassThreads - 1) / kPassThreads * 64;
+    const int64_t first = (int64_t)blockIdx.x * d.tile + (int64_t)w * per, lim = min(first + per, end);
+    uint32_t *row = rows[w];
+    auto load = [&](int64_t c0, uint32_t (&key)[kPassRegs]) {
+#pragma unroll
+        for (int k = 0; k < kPassRegs; ++k) {
+            const int64_t j = c0 + k * 64 + lane;
+            key[k] = j < lim ? d.keys[j] : 0u;
+        }
+    };
+    for (int64_t c0 = first; c0 < lim; c0 += kPassRegs * 64) {
+        uint32_t key[kPassRegs];
+        load(c0, key);
+#pragma unroll
+        for (int k = 0; k < kPassRegs; ++k)
+            if (c0 + k * 64 + lane < lim)
+                atomicAdd(&row[key[k] >> low], 1u);
+    }
     tile_bases(d, base, red, part);
     if (low && blockIdx.x == 0) {
-        for (int x = t; x < ndig; x += kSortThreads)
+        for (int x = t; x < ndig; x += kPassThreads)
             d.seg[x] = base[x];
         if (t == 0)
             d.seg[ndig] = (uint32_t)d.n;
     }
+    for (int x = t; x < ndig; x += kPassThreads)
+        wave_places(rows, x, base[x]);
+    __syncthreads();
     uint32_t *out = low ? d.vals_alt : d.vals;
-    const int64_t first = (int64_t)blockIdx.x * d.tile, lim = min(first + d.tile, (int64_t)d.n);
-    for (int64_t c0 = first; c0 < lim; c0 += kSortRegs * kSortThreads) {
-        uint32_t key[kSortRegs];
+    for (int64_t c0 = first; c0 < lim; c0 += kPassRegs * 64) {
+        uint32_t key[kPassRegs];
+        load(c0, key);
 #pragma unroll
-        for (int k = 0; k < kSortRegs; ++k) {
-            const int64_t j = c0 + k * kSortThreads + t;
-            key[k] = j < lim ? d.keys[j] : 0u;
-        }
-#pragma unroll
-        for (int k = 0; k < kSortRegs; ++k) {
-            if (c0 + k * kSortThreads >= lim)
-                break; // uniform over the workgroup
-            const int64_t j = c0 + k * kSortThreads + t;
+        for (int k = 0; k < kPassRegs; ++k) {
+            if (c0 + k * 64 >= lim)
+                break; // uniform over the wave
+            const int64_t j = c0 + k * 64 + lane;
             const bool valid = j < lim;
-            const uint32_t pos = round_place<kSortMaxDigits>(key[k] >> low, d.high_bits, valid, base, wcnt);
+            const uint32_t pos = round_place(key[k] >> low, d.high_bits, valid, row);
             if (valid && pos < (uint32_t)d.n) {
                 out[pos] = (uint32_t)j;
                 if (low)
@@ -220,57 +260,57 @@ __global__ __launch_bounds__(kSortThreads) void sort_first_pass_kernel(RandomOrd
     }
 }
 
-__global__ __launch_bounds__(kSortThreads) void sort_segment_kernel(RandomOrderDesc d)
+__global__ __launch_bounds__(kPassThreads) void sort_segment_kernel(RandomOrderDesc d)
 {
-    __shared__ uint32_t base[256];
-    __shared__ uint32_t wcnt[kSortWaves][256];
-    const int t = threadIdx.x, h = blockIdx.x;
-    const int ndig = 1 << d.high_bits, low = d.key_bits - d.high_bits, nlow = 1 << low;
+    __shared__ uint32_t rows[kPassWaves][256];
+    __shared__ uint32_t part[kPassWaves];
+    const int t = threadIdx.x, lane = t & 63, w = __builtin_amdgcn_readfirstlane(t >> 6), h = blockIdx.x;
+    const int low = d.key_bits - d.high_bits, nlow = 1 << low;
     const uint32_t lmask = (uint32_t)nlow - 1u;
     const uint32_t start = d.seg[h], end = d.seg[h + 1];
-    base[t] = 0;
-    for (int v = 0; v < kSortWaves; ++v)
-        wcnt[v][t] = 0;
+    for (int x = t; x < kPassWaves * 256; x += kPassThreads)
+        rows[0][x] = 0;
     __syncthreads();
-    for (uint32_t c0 = start; c0 < end; c0 += kSortRegs * kSortThreads) {
-        uint32_t key[kSortRegs];
+    // The wave's part of the segment.
+    const int64_t per = ((int64_t)end - start + kPassThreads - 1) / kPassThreads * 64;
+    const int64_t first = (int64_t)start + w * per, lim = min(first + per, (int64_t)end);
+    uint32_t *row = rows[w];
+    for (int64_t c0 = first; c0 < lim; c0 += kPassRegs * 64) {
+        uint32_t key[kPassRegs];
 #pragma unroll
-        for (int k = 0; k < kSortRegs; ++k) {
-            const uint32_t i = c0 + k * kSortThreads + t;
-            key[k] = i < end ? d.keys_alt[i] : 0u;
+        for (int k = 0; k < kPassRegs; ++k) {
+            const int64_t i = c0 + k * 64 + lane;
+            key[k] = i < lim ? d.keys_alt[i] : 0u;
         }
 #pragma unroll
-        for (int k = 0; k < kSortRegs; ++k)
-            if (c0 + k * kSortThreads + t < end)
-                atomicAdd(&base[key[k] & lmask], 1u);
+        for (int k = 0; k < kPassRegs; ++k)
+            if (c0 + k * 64 + lane < lim)
+                atomicAdd(&row[key[k] & lmask], 1u);
     }
     __syncthreads();
-    // Counts -> segment positions (an inclusive scan over the low digits, then shifted).
-    const uint32_t own = t < nlow ? base[t] : 0u;
-    for (int off = 1; off < nlow; off <<= 1) {
-        const uint32_t x = t < nlow && t >= off ? base[t - off] : 0u;
-        __syncthreads();
-        if (t < nlow)
-            base[t] += x;
-        __syncthreads();
-    }
+    uint32_t total = 0;
     if (t < nlow)
-        base[t] = start + base[t] - own;
-    __syncthreads();
-    for (uint32_t c0 = start; c0 < end; c0 += kSortRegs * kSortThreads) {
-        uint32_t key[kSortRegs], val[kSortRegs];
 #pragma unroll
-        for (int k = 0; k < kSortRegs; ++k) {
-            const uint32_t i = c0 + k * kSortThreads + t;
-            key[k] = i < end ? d.keys_alt[i] : 0u;
-            val[k] = i < end ? d.vals_alt[i] : 0u;
+        for (int v = 0; v < kPassWaves; ++v)
+            total += rows[v][t];
+    const uint32_t before = exclusive_scan(total, part);
+    if (t < nlow)
+        wave_places(rows, t, start + before);
+    __syncthreads();
+    for (int64_t c0 = first; c0 < lim; c0 += kPassRegs * 64) {
+        uint32_t key[kPassRegs], val[kPassRegs];
+#pragma unroll
+        for (int k = 0; k < kPassRegs; ++k) {
+            const int64_t i = c0 + k * 64 + lane;
+            key[k] = i < lim ? d.keys_alt[i] : 0u;
+            val[k] = i < lim ? d.vals_alt[i] : 0u;
         }
 #pragma unroll
-        for (int k = 0; k < kSortRegs; ++k) {
-            if (c0 + k * kSortThreads >= end)
-                break; // uniform over the workgroup
-            const bool valid = c0 + k * kSortThreads + t < end;
-            const uint32_t pos = round_place<256>(key[k] & lmask, low, valid, base, wcnt);
+        for (int k = 0; k < kPassRegs; ++k) {
+            if (c0 + k * 64 >= lim)
+                break; // uniform over the wave
+            const bool valid = c0 + k * 64 + lane < lim;
+            const uint32_t pos = round_place(key[k] & lmask, low, valid, row);
             if (valid && pos < end)
                 d.vals[pos] = val[k];
         }
@@ -357,8 +397,7 @@ void random_order_tiles(int n, int *tile, int *tiles)
     // Tiles of 4,096 samples, at most 256 of them (a whole multiple of 256 samples each).
     int64_t t = kRandomSortTile;
     if (((int64_t)n + t - 1) / t > kRandomSortMaxTiles)
-        t = (((int64_t)n + kRandomSortMaxTiles - 1) / kRandomSortMaxTiles + kSortThreads - 1) / kSortThreads *
-            kSortThreads;
+        t = (((int64_t)n + kRandomSortMaxTiles - 1) / kRandomSortMaxTiles + 255) / 256 * 256;
     *tile = (int)t;
     *tiles = (int)(((int64_t)n + t - 1) / t);
 }
@@ -398,9 +437,9 @@ hipError_t launch_random_order(const RandomOrderDesc &d, hipStream_t s, const ui
     RandomOrderDesc e = d;
     e.seg = d.counts + random_order_seg_offset(d.tiles, d.high_bits);
     hipLaunchKernelGGL(sort_count_kernel, dim3((unsigned)e.tiles), dim3(kSortThreads), 0, s, e);
-    hipLaunchKernelGGL(sort_first_pass_kernel, dim3((unsigned)e.tiles), dim3(kSortThreads), 0, s, e);
+    hipLaunchKernelGGL(sort_first_pass_kernel, dim3((unsigned)e.tiles), dim3(kPassThreads), 0, s, e);
     if (e.key_bits > e.high_bits)
-        hipLaunchKernelGGL(sort_segment_kernel, dim3(1u << e.high_bits), dim3(kSortThreads), 0, s, e);
+        hipLaunchKernelGGL(sort_segment_kernel, dim3(1u << e.high_bits), dim3(kPassThreads), 0, s, e);
     *order = e.vals;
     return hipGetLastError();
 }

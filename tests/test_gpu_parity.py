@@ -486,6 +486,15 @@ def test_random_sample_order_is_the_stable_bin_sort(lib, O, image, region):
     assert len(np.unique(key)) > 1
 
 
+@pytest.mark.parametrize("image,region", [(128, (63, 1)), (128, (577, 1)), (128, (1100, 1001)), (2112, (1100, 1001))],
+                         ids=["under-a-wave", "two-waves-of-eight", "long-tiles-one-pass", "long-tiles-two-pass"])
+def test_random_sample_order_wave_parts(lib, O, image, region):
+    """The sort's waves take contiguous parts of a tile or segment, 64 samples a round and eight
+    rounds of loads at a time: fewer samples than a wave, waves with no part, a last round of one
+    sample, and parts of more than eight rounds (tiles of 4,352 samples; 137 long segments)."""
+    test_random_sample_order_is_the_stable_bin_sort(lib, O, image, region)
+
+
 def test_train_step_accumulates(lib, O):
     """Two passes without an optimizer step add up (the zero-gradient contract)."""
     say("case: train accumulate")
