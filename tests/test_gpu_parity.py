@@ -178,6 +178,41 @@ def test_forward_coordinates_and_sizes(lib, O, shape, grids, filt, n, shift):
                      outs.view(np.float16).astype(np.float32), "outputs")
 
 
+@pytest.mark.parametrize("filt", [abi.NT_FILTER_BILINEAR, abi.NT_FILTER_CATMULL_ROM])
+def test_forward_grid_past_32_bit_texels(lib, filt):
+    """A grid of 65,536 x 65,544 texels (51.5 GB): its last eight rows, from texel 2^32 on, hold
+    1, all others 0. Footprints inside them sample 1, within the four corner products' and three
+    sums' fp16 roundings below 1 (2^-12 each)."""
+    import torch
+    say(f"case: forward large grid filter {filt}")
+    w, h, ch, n = 65536, 65544, 3, 256
+    if torch.cuda.mem_get_info()[0] < 56 << 30:
+        pytest.skip("needs 52 GB of device memory")
+    rng = np.random.default_rng(5)
+    values = torch.zeros(w * h * ch, dtype=torch.float32, device="cuda")
+    values[(h - 8) * w * ch:] = 1.0
+    grids = [P.Grid(w, h, 1, ch, values=values)]
+    grids += [P.make_grid(4, 4, 1, ch, rng, with_adam=False).converted(True, "cuda") for _ in range(3)]
+    net = P.make_network(SHAPES["ref"]["sizes"], rng=rng, init="xavier").converted(True, "cuda")
+    lat = abi.nt_latents()
+    lat.num_grids, lat.channels = 4, ch
+    for i, g in enumerate(grids):
+        lat.grids[i] = g.struct()
+    uvz = np.zeros((n, 3), np.float32)
+    uvz[:, 0] = rng.uniform(0, 1, n)
+    uvz[:, 1] = (h - rng.uniform(3, 5, n)) / h  # rows h - 7 .. h - 1
+    guvz = torch.from_numpy(uvz).cuda()
+    feats = torch.zeros(n * 12, dtype=torch.int16, device="cuda")
+    outs = torch.zeros(n * 16, dtype=torch.int16, device="cuda")
+    nt.check(lib.nt_forward(C.byref(lat), C.byref(net.struct()), filt, guvz.data_ptr(), n, feats.data_ptr(),
+                            outs.data_ptr(), None))
+    sync()
+    got = feats.cpu().numpy().view(np.float16).astype(np.float32).reshape(n, 12)[:, :3]
+    del values, grids
+    torch.cuda.empty_cache()
+    assert np.max(np.abs(got - 1.0)) <= 8 * 2.0 ** -12
+
+
 # ---- the fused train step -----------------------------------------------------------------
 
 TRAIN_CASES = [
