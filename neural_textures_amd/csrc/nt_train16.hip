@@ -1029,6 +1029,7 @@ __device__ __forceinline__ void scatter_path(const Train16Desc &d, const Grid16 
             asm("v_pk_max_u16 %0, %1, %2" : "=v"(top) : "v"(top), "v"(b));
         }
     const bool finite = __ballot((top & 0xFFFFu) >= 0x7C00u || (top >> 16) >= 0x7C00u) == 0;
+    wave_sync(); // the dX0 rows, written by the wave's other lanes and read transposed below
     Footprint f[J];
     int mnx[J], mny[J], mxx[J], mxy[J]; // row minima of x0, y0, -x0, -y0
 #pragma unroll
