@@ -152,12 +152,14 @@ hipError_t launch_random_order(const RandomOrderDesc &d, hipStream_t s, const ui
 constexpr int kRandomPathTile = 1024;
 hipError_t launch_random_path(const RandomOrderDesc &d, hipStream_t s);
 
-// The bin-ordered random-texel kernel's scatter: each wave's weight rows (32 samples, hi and
-// lo, kPathCells cells a pass) in rows of kPathStride halves (an odd number of 8-byte chunks:
-// rows fall in distinct LDS banks).
-constexpr int kPathCells = 64;
-constexpr int kPathStride = kPathCells + 4;
+// The bin-ordered random-texel kernel's scatter: each wave's weight rows (32 samples, three
+// halves a weight, path_cells cells a pass) in rows of path_stride halves (an odd number of
+// 16-byte chunks: each lane clears rows of its own with 16-byte stores, which then fall in
+// distinct LDS banks). Two groups of four grids have room for 32 cells.
+constexpr int path_cells(int grids, int groups) { return grids == 4 && groups == 2 ? 32 : 64; }
+constexpr int path_stride(int grids, int groups) { return path_cells(grids, groups) + 8; }
 constexpr int kPathMaxCells = 256; // a larger cell box takes per-sample atomics
+constexpr float kPathMinWeight = 0x1p-27f; // three halves no longer hold a smaller corner weight
 
 struct Train16Desc {
     Grid16 grid[NT_MAX_GRIDS];

@@ -439,6 +439,54 @@ def test_random_texel_path_scatter(lib, O, shape, image, n, overflow):
 
 
 @pytest.mark.parametrize("shape", ["c2", "c4"])
+@pytest.mark.parametrize("size,grid_sizes", [
+    # left-clamped samples of a five-texel image: t = 0.1f * 5 - 0.5 = 2^-27 on a grid as wide, so
+    # that corners' weights go down to 2^-27 times the row's fraction
+    ((5, 64), [(5, 60), (20, 20), (7, 31), (33, 5)]),
+    ((64, 64), [(20, 20), (13, 29), (5, 60), (31, 9)]),
+])
+@pytest.mark.parametrize("loss_weight", [1.0, 2.0 ** -22], ids=["", "subnormal-gradients"])
+def test_random_texel_path_scatter_weights(lib, shape, size, grid_sizes, loss_weight):
+    """The bin-ordered scatter holds corner weights as precisely as slot order's fp32 products,
+    down to the smallest: all weights, inputs and errors of one sign, so that every term of a
+    texel's sum has one sign, and two orders of the at most 64 terms (64 samples) agree within
+    64 roundings of 2^-24 each and the products'. Texels that a tiny corner alone reaches
+    included."""
+    say(f"case: path scatter weights {shape} {size} loss weight {loss_weight}")
+    w, h = size
+    rng = np.random.default_rng(w)
+    st = make_state(shape, image=64, region=(64, 1), seed=5)
+    st.sample_mode = abi.NT_SAMPLES_RANDOM
+    st.image_width, st.image_height = w, h
+    st.textures = [P.make_texture(w, h, c, np.full((h, w, 4), 100.0, np.float32)) for c in SHAPES[shape]["tex"]]
+    for t in st.textures:
+        t.loss_weight = loss_weight
+    st.grids = [P.make_grid(gw, gh, 1, 16, rng) for gw, gh in grid_sizes[:len(SHAPES[shape]["grids"])]]
+    for g in st.grids:
+        g.values = np.abs(g.values) + np.float32(0.01)
+    for l in range(st.net.num_layers):
+        st.net.weights[l] = P.f16_bits(np.abs(st.net.weights[l].view(np.float16).astype(np.float32)) * 0.25)
+    grads = []
+    for flags in (0, abi.NT_HOOK_SORT_RANDOM):
+        gs = st.to_torch()
+        nt.check(lib.nt_set_test_hooks(0, flags))
+        try:
+            gs = gpu_workspace(lib, gs, 0)
+            nt.check(lib.nt_train_step(C.byref(gs.params()), 0, None))
+            sync()
+        finally:
+            nt.check(lib.nt_set_test_hooks(0, 0))
+        grads.append([to_np(g.grads).astype(np.float64) for g in gs.grids])
+    tiny = 0
+    for want, got in zip(*grads):
+        assert np.all(want <= 0) and np.any(want < 0)
+        assert np.array_equal(got == 0, want == 0)
+        assert np.max(np.abs(got - want) / np.where(want == 0, 1, -want)) <= 66 * 2.0 ** -24
+        tiny += np.count_nonzero((want < 0) & (want > 2.0 ** -24 * want.min()))
+    assert tiny > 0 or w != 5
+
+
+@pytest.mark.parametrize("shape", ["c2", "c4"])
 @pytest.mark.parametrize("image,n,max_wg", [(64, 127, 0), (64, 129, 1), (64, 640, 2), (64, 1300, 2), (512, 1300, 2),
                                             (64, 2100, 3)])
 def test_train_step_random_tiles(lib, O, shape, image, n, max_wg):
