@@ -247,9 +247,13 @@ int64_t nt_mip_chain_layout(int width, int height, int num_mips, int64_t *mip_of
 /* The same for 4x4 block storage (blocks per dimension = max(size>>2, 1), train.cu:220). */
 int64_t nt_block_chain_layout(int width, int height, int num_mips, int64_t *block_offset);
 /* Bytes of scratch nt_train_step needs for these parameters (0 on error); also enough for
- * nt_inference's fixed-order SSE. A NT_SAMPLES_RANDOM step of 262,144 samples or more (65,536
- * where there is a sample to at most 32 image texels) also holds its sample sort (keys, sample
- * indices and per-tile counts, ~12 bytes a sample). */
+ * nt_inference's fixed-order SSE. With the other fields equal they never fall as the region
+ * grows in width or height, or the samples of NT_SAMPLES_RANDOM in number, so a workspace of
+ * the largest step's bytes holds every smaller one's. A NT_SAMPLES_RANDOM step of 65,536
+ * samples or more reserves its sample sort (keys, sample indices and per-tile counts, ~12 bytes
+ * a sample), whether or not the image's size has it sort. A step given fewer bytes runs wider
+ * tiles and, below 262,144 samples, without the sort, if they hold that (the same results up to
+ * the order of fp32 sums), else fails with NT_ERR_WORKSPACE. */
 size_t nt_train_workspace_bytes(const nt_params *params, nt_kernel_type type);
 
 /* Profiling hook (no reference counterpart): the next nt_train_step, nt_optimize_latents,

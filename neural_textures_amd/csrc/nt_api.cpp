@@ -330,7 +330,9 @@ struct TrainPlan {
     size_t weight_bytes;
     int fp_w[NT_MAX_GRIDS], fp_h[NT_MAX_GRIDS], fp_off[NT_MAX_GRIDS], vb_off[NT_MAX_GRIDS];
     int cb_w[NT_MAX_GRIDS], cb_h[NT_MAX_GRIDS], w_row0[NT_MAX_GRIDS];
-    size_t lds, workspace;
+    // workspace: the bytes this plan uses; reserve: at least that, and never less for a larger
+    // step (nt_train_workspace_bytes).
+    size_t lds, workspace, reserve;
     // The 16-channel unconstrained kernel (nt_train16.hip), when it applies.
     int use16, groups, rows;
     Train16Desc t16;
@@ -360,7 +362,11 @@ float pow2_reciprocal(int n)
     return n > 0 && (n & (n - 1)) == 0 ? 1.f / (float)n : 0.f;
 }
 
-void plan16(const nt_params *p, nt_kernel_type type, TrainPlan *plan, bool bc6_inner_step)
+// Flags of plan_train: the inner step of the BC6 phase; the plan of least workspace (tiles of
+// four chunks, two groups for random texels, no sort below kRandomSortMinSamples).
+enum { kPlanBc6Inner = 1, kPlanSmall = 2 };
+
+void plan16(const nt_params *p, nt_kernel_type type, TrainPlan *plan, int flags)
 {
     plan->use16 = 0;
     const bool random = p->sample_mode == NT_SAMPLES_RANDOM;
@@ -376,7 +382,7 @@ void plan16(const nt_params *p, nt_kernel_type type, TrainPlan *plan, bool bc6_i
     int cap = device_cu_count();
     if (const int hook = g_hook_max_workgroups.load(std::memory_order_relaxed); hook > 0)
         cap = std::min(cap, hook);
-    if (random && NG == 2 &&
+    if (random && NG == 2 && !(flags & kPlanSmall) &&
         (p->num_samples <= kChunk * cap ||
          (plan->shape == kShapeC4 && 8 * (int64_t)p->num_samples <= texels)))
         NG = 1;
@@ -454,6 +460,7 @@ void plan16(const nt_params *p, nt_kernel_type type, TrainPlan *plan, bool bc6_i
     // two); the reference network at 509 x 331, 168 tiles of four on 256 CUs, 76.8 -> 69.2 us
     // (three). Equal counts keep the wider tile (fewer halo texels and box flushes).
     d.groups = NG;
+    int64_t reserve_rows = 0;
     {
         int64_t best = 0;
         for (int tc = 4; tc >= 1; tc /= 2) {
@@ -464,11 +471,14 @@ void plan16(const nt_params *p, nt_kernel_type type, TrainPlan *plan, bool bc6_i
             if (n > (1 << 30) || (best > 0 && serial >= best))
                 continue;
             // A region step with the dense optimizer and fewer than 16 wide tiles keeps them, and
-            // with them its workspace of one gradient row per 64 x 8NG tile, which callers of
-            // such steps size their memory by; an update-log or block-record step's workspace
-            // holds a row per workgroup.
-            if (best > 0 && !random && !bc6_inner_step && p->latent_update == NT_LATENT_DENSE && d.ntiles < 16)
+            // with them a workspace of exactly one gradient row per 64 x 8NG tile: its size has
+            // been that since before there were narrow tiles. This costs such steps speed (two
+            // grids at 64 x 32 samples: 44.8 us, 21.5 with an update log).
+            if (best > 0 && ((flags & kPlanSmall) || (!random && !(flags & kPlanBc6Inner) &&
+                                                      p->latent_update == NT_LATENT_DENSE && d.ntiles < 16))) {
+                reserve_rows = d.ntiles;
                 break;
+            }
             best = serial;
             d.tile_chunks = tc;
             d.tiles_x = (int)tx;
@@ -478,6 +488,12 @@ void plan16(const nt_params *p, nt_kernel_type type, TrainPlan *plan, bool bc6_i
             return;
     }
     d.nwg = std::min(d.ntiles, cap);
+    // A narrower tile for a smaller or raggeder step may take more workgroups than a larger
+    // step's wide tiles, so the reserved rows are those of one-chunk tiles, which only grow.
+    if (reserve_rows == 0)
+        reserve_rows = random ? ((int64_t)p->num_samples + kChunk - 1) / kChunk
+                              : (int64_t)((rw + kChunkW - 1) / kChunkW) * ((rows + kChunkH * NG - 1) / (kChunkH * NG));
+    reserve_rows = std::min<int64_t>(reserve_rows, cap);
     d.xcd_per = (d.ntiles % 8 == 0 && d.nwg % 8 == 0) ? d.ntiles / 8 : 0;
     // Margin of the chunk cell box beyond the cells positions can reach. A test hook drops
     // it, to drive the scatter's out-of-box path (per-sample global atomics), which
@@ -643,6 +659,7 @@ void plan16(const nt_params *p, nt_kernel_type type, TrainPlan *plan, bool bc6_i
     plan->rows = d.nwg; // the groups of a workgroup merge their partials in LDS
     plan->weight_bytes = 0; // each workgroup builds its weight image in LDS
     plan->workspace = (size_t)plan->rows * (size_t)plan->P * sizeof(float);
+    plan->reserve = std::max<size_t>(plan->rows, reserve_rows) * (size_t)plan->P * sizeof(float);
     // Random texels: the sort of the sample indices by bin after the partial rows (keys and
     // sample indices in two buffers each, then the per-tile digit counts). From 262,144
     // samples (two grids, 2048^2 texels: 231 -> 187 us a step; four, a million of 4096^2: 1,268
@@ -651,8 +668,16 @@ void plan16(const nt_params *p, nt_kernel_type type, TrainPlan *plan, bool bc6_i
     // 241 sorted; fewer, 32,768 of 1024^2: 71, 82 sorted).
     plan->sort_off = plan->sort_temp = 0;
     const bool sorted = p->num_samples >= kRandomSortMinSamples ||
-                        (p->num_samples >= kRandomSortMinDense && 32 * (int64_t)p->num_samples >= texels) ||
+                        (p->num_samples >= kRandomSortMinDense && 32 * (int64_t)p->num_samples >= texels &&
+                         !(flags & kPlanSmall)) ||
                         g_hook_sort_random.load(std::memory_order_relaxed);
+    const size_t n = (size_t)p->num_samples;
+    const size_t keys = (n * 2 + 255) & ~(size_t)255, vals = (n * 4 + 255) & ~(size_t)255;
+    // Its counts depend on the image's bins, and whether there is a sort on its size: reserved
+    // for any image.
+    if (random && p->num_samples >= kRandomSortMinDense)
+        plan->reserve = ((plan->reserve + 255) & ~(size_t)255) + 2 * keys + 2 * vals +
+                        ((random_order_count_bytes_bound() + 255) & ~(size_t)255);
     if (random && sorted) {
         // Bins of 64 x 64 texels (coarser ones, one 8-bit sort pass, gained less).
         const int shift = 6;
@@ -663,9 +688,7 @@ void plan16(const nt_params *p, nt_kernel_type type, TrainPlan *plan, bool bc6_i
             int bits = 1;
             while ((1 << bits) < bx * by)
                 ++bits;
-            const size_t n = (size_t)p->num_samples;
             const size_t temp = (random_order_count_bytes(p->num_samples, bits) + 255) & ~(size_t)255;
-            const size_t keys = (n * 2 + 255) & ~(size_t)255, vals = (n * 4 + 255) & ~(size_t)255;
             plan->sort_off = (plan->workspace + 255) & ~(size_t)255;
             plan->sort_temp = temp;
             plan->sort_bins_x = bx;
@@ -673,6 +696,7 @@ void plan16(const nt_params *p, nt_kernel_type type, TrainPlan *plan, bool bc6_i
             plan->workspace = plan->sort_off + 2 * keys + 2 * vals + temp;
         }
     }
+    plan->reserve = std::max(plan->reserve, plan->workspace);
     d.image_w = p->image_width;
     d.image_h = p->image_height;
     d.off_x = p->texel_offset_x;
@@ -725,13 +749,13 @@ nt_params bc6_inner(const nt_params *p, const TrainPlan &plan, uint8_t *ws)
     return q;
 }
 
-int plan_train(const nt_params *p, nt_kernel_type type, TrainPlan *plan, bool bc6_inner_step = false);
+int plan_train(const nt_params *p, nt_kernel_type type, TrainPlan *plan, int flags = 0);
 
 // The BC6 block phase (NT_BLOCK_FEATURES, NT_FINALIZE) runs an unconstrained train step on
 // texels expanded from the block records of every level a sample reaches (Bc6PhaseDesc):
 // the step is planned as one over grids whose texels live in the workspace, after its own
 // scratch. Sets plan->bc6 (and then the inner step's plan), or leaves the plan alone.
-void plan_bc6_phase(const nt_params *p, TrainPlan *plan)
+void plan_bc6_phase(const nt_params *p, TrainPlan *plan, int flags)
 {
     plan->bc6 = 0;
     const int C = p->latents.channels, G = p->latents.num_grids;
@@ -755,7 +779,7 @@ void plan_bc6_phase(const nt_params *p, TrainPlan *plan)
     }
     const nt_params q = bc6_inner(p, t, nullptr);
     TrainPlan inner;
-    if (plan_train(&q, NT_UNCONSTRAINED, &inner, true) != NT_OK)
+    if (plan_train(&q, NT_UNCONSTRAINED, &inner, flags | kPlanBc6Inner) != NT_OK)
         return;
     // The inner plan, with the phase's fields.
     for (int gi = 0; gi < G; ++gi)
@@ -805,12 +829,13 @@ void plan_bc6_phase(const nt_params *p, TrainPlan *plan)
         first += ((int64_t)x.nbx * x.nby + kBc6PhaseBlocks - 1) / kBc6PhaseBlocks * kBc6PhaseBlocks;
     }
     b.total_blocks = first;
+    inner.reserve = ((inner.reserve + 255) & ~(size_t)255) + (off - ((inner.workspace + 255) & ~(size_t)255));
     inner.workspace = off;
     inner.bc6 = 1;
     *plan = inner;
 }
 
-int plan_train(const nt_params *p, nt_kernel_type type, TrainPlan *plan, bool bc6_inner_step)
+int plan_train(const nt_params *p, nt_kernel_type type, TrainPlan *plan, int flags)
 {
     if (!p)
         return fail(NT_ERR_NULL_POINTER, "params is NULL");
@@ -851,7 +876,7 @@ int plan_train(const nt_params *p, nt_kernel_type type, TrainPlan *plan, bool bc
     plan->nwg = plan->tiles_x * tiles_y;
     plan->P = train_grad_total(shape);
     plan->weight_bytes = train_weight_bytes(shape);
-    plan->workspace = plan->weight_bytes + (size_t)plan->nwg * (size_t)plan->P * sizeof(float);
+    plan->workspace = plan->reserve = plan->weight_bytes + (size_t)plan->nwg * (size_t)plan->P * sizeof(float);
 
     // LDS footprint box per grid: every texel a 64 x 8 block of positions can touch (the
     // bilinear corners of positions in [x, x + 64] span at most ceil(64 r) + 2 texels, plus
@@ -938,13 +963,36 @@ int plan_train(const nt_params *p, nt_kernel_type type, TrainPlan *plan, bool bc
     }
     plan->rows = plan->nwg;
     plan->bc6 = 0;
-    plan16(p, type, plan, bc6_inner_step);
+    plan16(p, type, plan, flags);
     if (type != NT_UNCONSTRAINED)
-        plan_bc6_phase(p, plan);
+        plan_bc6_phase(p, plan, flags);
     if (type != NT_UNCONSTRAINED && !plan->bc6)
         return fail(NT_ERR_UNSUPPORTED, "block records train through the BC6 phase, built for 3, 8 and 16 "
                                         "channels");
     return NT_OK;
+}
+
+// plan_train, or where `bytes` of scratch do not hold that plan, the one of least workspace if
+// they hold it (narrow tiles and the sort of fewer samples are for speed only: a caller with as
+// much scratch as four-chunk tiles need runs those). The caller compares plan->workspace.
+int plan_within(const nt_params *p, nt_kernel_type type, size_t bytes, TrainPlan *plan)
+{
+    const int st = plan_train(p, type, plan);
+    if (st != NT_OK || plan->workspace <= bytes)
+        return st;
+    TrainPlan small;
+    if (plan_train(p, type, &small, kPlanSmall) == NT_OK && small.workspace <= bytes)
+        *plan = small;
+    return NT_OK;
+}
+
+// The scratch of params->workspace that a train step may use: all but the update log.
+size_t scratch_bytes(const nt_params *p)
+{
+    if (!p || !p->workspace)
+        return 0;
+    const size_t mb = touched_bytes(p);
+    return mb == 0 ? p->workspace_bytes : p->workspace_bytes > mb ? (p->workspace_bytes - mb) & ~(size_t)255 : 0;
 }
 
 } // namespace
@@ -1044,7 +1092,7 @@ size_t nt_train_workspace_bytes(const nt_params *params, nt_kernel_type type)
         return 0;
     // Large enough for nt_inference's fixed-order SSE partials too; the update log of
     // NT_LATENT_TOUCHED after both.
-    const size_t base = std::max(plan.workspace, nt_inference_workspace_bytes(params));
+    const size_t base = std::max(plan.reserve, nt_inference_workspace_bytes(params));
     const size_t mb = touched_bytes(params);
     return mb ? ((base + 255) & ~(size_t)255) + mb : base;
 }
@@ -1340,7 +1388,7 @@ extern "C" {
 int nt_train_step(const nt_params *p, nt_kernel_type type, void *stream)
 {
     TrainPlan plan;
-    int st = plan_train(p, type, &plan);
+    int st = plan_within(p, type, scratch_bytes(p), &plan);
     if (st)
         return st;
     const size_t mb = touched_bytes(p);
@@ -1356,7 +1404,7 @@ int nt_train_step(const nt_params *p, nt_kernel_type type, void *stream)
 int nt_random_sample_order(const nt_params *p, uint32_t *order, void *stream)
 {
     TrainPlan plan;
-    int st = plan_train(p, NT_UNCONSTRAINED, &plan);
+    int st = plan_within(p, NT_UNCONSTRAINED, scratch_bytes(p), &plan);
     if (st)
         return st;
     if (!order)
@@ -1386,7 +1434,7 @@ size_t nt_train_static_scratch_bytes(void) { return kStaticScratchBytes; }
 int nt_train_step_static(const nt_params *p, nt_kernel_type type, void *stream)
 {
     TrainPlan plan;
-    int st = plan_train(p, type, &plan);
+    int st = plan_within(p, type, kStaticScratchBytes, &plan);
     if (st)
         return st;
     if (p->latent_update != NT_LATENT_DENSE)
@@ -1562,7 +1610,7 @@ int nt_optimize_latents(const nt_params *p, nt_kernel_type type, void *stream)
 int nt_train_iteration(const nt_params *p, nt_kernel_type type, void *stream)
 {
     TrainPlan plan;
-    int st = plan_train(p, type, &plan);
+    int st = plan_within(p, type, scratch_bytes(p), &plan);
     if (st)
         return st;
     const size_t mb = touched_bytes(p);

@@ -145,6 +145,7 @@ void random_order_tiles(int n, int *tile, int *tiles);
 int random_order_high_bits(int key_bits, int tiles);
 // Bytes of the per-tile digit counts for n samples and keys of key_bits bits.
 size_t random_order_count_bytes(int n, int key_bits);
+size_t random_order_count_bytes_bound(); // ... for any n and key_bits
 // Bins, then the stable sort; *order is the sorted sample indices (d.vals).
 hipError_t launch_random_order(const RandomOrderDesc &d, hipStream_t s, const uint32_t **order);
 // ... and each tile of kRandomPathTile of its entries (the train kernel's tiles) reordered in

@@ -427,6 +427,13 @@ size_t random_order_count_bytes(int n, int key_bits)
     return random_order_seg_offset(tiles, high) * sizeof(uint32_t) + (ndig + 1) * sizeof(uint32_t);
 }
 
+size_t random_order_count_bytes_bound()
+{
+    // One pass: at most 64 Ki counts; two: 256 digits of at most 256 tiles.
+    static_assert(256 * kRandomSortMaxTiles <= 65536, "two-pass counts");
+    return 65536 * sizeof(uint32_t) + (kSortMaxDigits + 1) * sizeof(uint32_t);
+}
+
 hipError_t launch_random_order(const RandomOrderDesc &d, hipStream_t s, const uint32_t **order)
 {
     int tile, tiles;

@@ -158,6 +158,99 @@ def test_config_shapes_plan_the_16_channel_kernel(lib, shape, ng, margins):
         assert lib.nt_set_test_hooks(0, 0) == 0
 
 
+def _need(lib, st, ktype=0):
+    need = lib.nt_train_workspace_bytes(C.byref(st.params()), ktype)
+    assert need > 0, lib.nt_last_error()
+    return need
+
+
+def _region(st, w, h, update=abi.NT_LATENT_DENSE):
+    st.region_width, st.num_samples, st.latent_update = w, w * h, update
+    return st
+
+
+@pytest.mark.parametrize("shape", ["c2", "c4", "ref16", "ref16f"])
+@pytest.mark.parametrize("update,blocks", [(abi.NT_LATENT_DENSE, False), (abi.NT_LATENT_TOUCHED, False),
+                                           (abi.NT_LATENT_DENSE, True)])
+def test_workspace_grows_with_the_region(lib, shape, update, blocks):
+    """A workspace sized for a region holds every smaller one's step: the bytes never fall as a
+    region grows in width or height, whatever tiles each size takes."""
+    from helpers import make_state
+    st = make_state(shape, image=256, blocks=blocks)
+    ktype = abi.NT_BLOCK_FEATURES if blocks else abi.NT_UNCONSTRAINED
+    sizes = [1, 15, 16, 17, 33, 64, 65, 100, 160, 161, 208, 255, 256, 331, 400, 509, 512, 700, 1024]
+    need = np.array([[_need(lib, _region(st, w, h, update), ktype) for h in sizes] for w in sizes])
+    assert np.all(np.diff(need, axis=0) >= 0) and np.all(np.diff(need, axis=1) >= 0)
+
+
+@pytest.mark.parametrize("shape", ["c2", "c4"])
+def test_workspace_grows_with_random_samples(lib, shape):
+    """The same for random texels: over sample counts (groups, tile widths, sort) at each image
+    size, and over image sizes from the sort's least count up."""
+    from helpers import make_state
+    st = make_state(shape, image=256)
+    st.sample_mode = abi.NT_SAMPLES_RANDOM
+    counts = [1, 127, 128, 129, 4096, 16384, 32767, 32768, 32769, 65535, 65536, 65537, 100000, 262143, 262144, 262145,
+              266241, 1 << 20, (1 << 20) + 1, 3 << 20]
+    need = []
+    for image in (64, 512, 1448, 2048, 4096, 8192, 16384, 20000):
+        st.image_width = st.image_height = image
+        for t in st.textures:
+            t.width = t.height = image
+        need.append([_need(lib, _region(st, n, 1)) for n in counts])
+    need = np.array(need)
+    assert np.all(np.diff(need, axis=1) >= 0)
+    assert np.all(np.diff(need[:, counts.index(65536):], axis=0) >= 0)
+
+
+@pytest.mark.parametrize("shape,ng,w,h,mode,blocks", [
+    ("c2", 2, 509, 331, abi.NT_SAMPLES_REGION, False), ("c4", 1, 300, 217, abi.NT_SAMPLES_REGION, False),
+    ("ref16", 2, 509, 331, abi.NT_SAMPLES_REGION, False), ("c4", 1, 256, 256, abi.NT_SAMPLES_REGION, True),
+    ("c2", 2, 16384, 1, abi.NT_SAMPLES_RANDOM, False), ("c4", 2, 100000, 1, abi.NT_SAMPLES_RANDOM, False),
+])
+def test_workspace_of_wide_tiles_is_enough(lib, shape, ng, w, h, mode, blocks):
+    """A step is not refused for want of the speed-only scratch (rows of narrow tiles, the sort
+    of fewer than 262,144 samples): a row per workgroup of four-chunk tiles is enough, 16 bytes
+    less is not. The argument after the workspace in nt_train_iteration's checks is invalid, so
+    nothing is launched."""
+    from helpers import make_state
+    st = _region(make_state(shape, image=256, blocks=blocks), w, h)
+    st.sample_mode = mode
+    ktype = abi.NT_BLOCK_FEATURES if blocks else abi.NT_UNCONSTRAINED
+    pads = [abi.pad16(s) for s in st.net.sizes]
+    row = 4 * sum(pads[l + 1] * pads[l] + pads[l + 1] for l in range(len(pads) - 1))
+    tiles = -(-w // (512 * ng)) if mode == abi.NT_SAMPLES_RANDOM else -(-w // 64) * -(-h // (8 * ng))
+    least = min(tiles, 256) * row
+    if blocks:
+        least = -(-least // 256) * 256 + sum(2 * -(-g.width * g.height * g.channels * 4 // 256) * 256 for g in st.grids)
+    assert _need(lib, st, ktype) > least
+    p = st.params()
+    p.mlp.weight_moment1[0] = None
+    ws = np.zeros(least + 16, np.uint8)
+    p.workspace = C.c_void_p((ws.ctypes.data + 15) // 16 * 16)
+    for size, want in ((least, abi.NT_ERR_NULL_POINTER), (least - 16, abi.NT_ERR_WORKSPACE)):
+        p.workspace_bytes = size
+        assert lib.nt_train_iteration(C.byref(p), ktype, None) == want, lib.nt_last_error()
+
+
+def test_static_step_takes_the_smaller_plan(lib):
+    """nt_train_step_static is not refused either where only the wide tiles' rows fit its scratch
+    (block phase, four grids whose expanded chains leave 12 MB of the 32 MiB: 256 narrow tiles
+    need 14.9 MB of rows, 128 wide ones half). Without a device the launch is what fails."""
+    import torch
+    if torch.cuda.is_available():
+        pytest.skip("would launch over host buffers")
+    from helpers import make_state
+    st = _region(make_state("c4", image=256, blocks=True), 256, 256)
+    for g, (w, h) in zip(st.grids, [(400, 384), (64, 200), (32, 32), (16, 16)]):
+        g.width, g.height, g.num_mips = w, h, 1
+    p = st.params()
+    p.workspace = None
+    need = _need(lib, st, abi.NT_BLOCK_FEATURES)
+    assert need > lib.nt_train_static_scratch_bytes()
+    assert lib.nt_train_step_static(C.byref(p), abi.NT_BLOCK_FEATURES, None) == abi.NT_ERR_HIP, lib.nt_last_error()
+
+
 def test_random_sample_order_refusals(lib):
     """nt_random_sample_order refuses, before touching a device, parameters that train in
     slot order (random texels below the sort's sample count without the hook, region

@@ -364,6 +364,31 @@ def test_train_step_tile_widths(lib, O, shape, rows, max_wg, ragged):
     check_train_grads(st, gs, alt)
 
 
+@pytest.mark.parametrize("shape,region,mode,tiles", [
+    ("c2", (256, 64), abi.NT_SAMPLES_REGION, 16), ("ref16", (250, 61), abi.NT_SAMPLES_REGION, 16),
+    ("c2", (2048, 1), abi.NT_SAMPLES_RANDOM, 2), ("c4", (1100, 1), abi.NT_SAMPLES_RANDOM, 2),
+])
+def test_train_step_within_wide_tiles_workspace(lib, O, shape, region, mode, tiles):
+    """A workspace of one gradient row per four-chunk tile (fewer bytes than narrow tiles take)
+    runs those: gradients as the oracle's, nothing written past it."""
+    import torch
+    say(f"case: small workspace {shape} {region} mode {mode}")
+    st = make_state(shape, image=256, region=region, seed=9)
+    st.sample_mode = mode
+    alt, gs = st.converted(False), st.to_torch()
+    oracle_step(O, st, 0)
+    oracle_step(O, alt, 0, accum_f32=True)
+    pads = [abi.pad16(x) for x in st.net.sizes]
+    least = tiles * 4 * sum(pads[l + 1] * pads[l] + pads[l + 1] for l in range(len(pads) - 1))
+    assert lib.nt_train_workspace_bytes(C.byref(gs.params()), 0) > least
+    whole = torch.full((least + 65536,), 0xA5, dtype=torch.uint8, device="cuda")
+    gs.workspace = whole[:least]
+    nt.check(lib.nt_train_step(C.byref(gs.params()), 0, None))
+    sync()
+    assert bool((whole[least:] == 0xA5).all())
+    check_train_grads(st, gs, alt)
+
+
 @pytest.mark.parametrize("shape,region,max_wg,flags,image", [
     ("ref", (64, 32), 0, 0, 128), ("c1", (64, 32), 0, 0, 128), ("c2", (64, 32), 0, 0, 128),
     ("c4", (64, 32), 0, 0, 128), ("c2", (50, 13), 2, 0, 128), ("c4", (100, 7), 1, 0, 128),
