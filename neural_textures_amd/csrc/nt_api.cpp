@@ -372,20 +372,30 @@ void plan16(const nt_params *p, nt_kernel_type type, TrainPlan *plan, int flags)
     const bool random = p->sample_mode == NT_SAMPLES_RANDOM;
     const int64_t texels = (int64_t)p->image_width * p->image_height;
     int NG = train16_groups(plan->shape, random);
-    // Random texels run one group of four waves a workgroup instead of two where that puts every
-    // 128 samples on a CU of their own (up to 32,768 on 256 CUs: two grids at 16,384 samples
-    // 39.3 -> 32.2 us, four 153 -> 135), and four grids also where the samples are sparse, at
-    // most one to eight texels: the taps then come from HBM, and the one group, with registers
-    // to issue them at the start of a chunk, waits for them less (four grids, a million samples
-    // of 4096^2 texels: 872 -> 823 us; of 2048^2, one to four texels: 579 -> 619).
+    // Random texels run two groups of four waves a workgroup, or one. One group takes c = samples /
+    // (128 CUs), rounded up, chunks in sequence, two take ceil(c / 2) of about twice the time in
+    // sparse images and 1.7 times in dense ones. So one group where c is 1 (two grids at 16,384
+    // samples 37.2 -> 31.8 us, at 40,960, c = 2, 50.5 two groups, 52.7 one; four 79 -> 70), and with
+    // four grids where two would idle one of theirs: c = 3 (66,048 to 98,304 samples: 1.02 to 1.20
+    // times as fast at any density, 229,376 of one to three texels, c = 7, 157 two groups, 182 one),
+    // and any odd c in an image of 12 texels a sample or more, where the taps come from HBM and the
+    // one group, with registers to issue them at the start of a chunk, waits for them less (163,840
+    // samples, 16 texels: 169 -> 164 us, 8 texels 149 two groups, 152 one; 131,072, c = 4, 16
+    // texels: 133 two groups, 138 one). That carries even c too from kRandomSortMinSamples samples
+    // (a million, 16 texels: 861 -> 840 us, 12: 767 -> 759, 8: 670 two groups, 690 one, 4: 557 and
+    // 633; 262,144, 16 texels: 241 -> 238, 12: 209 both, 11: 199 two groups, 208 one).
     // (A test hook can lower the workgroups, so that small steps loop and take two groups.)
     int cap = device_cu_count();
     if (const int hook = g_hook_max_workgroups.load(std::memory_order_relaxed); hook > 0)
         cap = std::min(cap, hook);
-    if (random && NG == 2 && !(flags & kPlanSmall) &&
-        (p->num_samples <= kChunk * cap ||
-         (plan->shape == kShapeC4 && 8 * (int64_t)p->num_samples <= texels)))
-        NG = 1;
+    if (random && NG == 2 && !(flags & kPlanSmall)) {
+        const int64_t chunks = ((int64_t)p->num_samples + kChunk * cap - 1) / (kChunk * cap);
+        const bool sparse = 12 * (int64_t)p->num_samples <= texels;
+        if (chunks == 1 ||
+            (plan->shape == kShapeC4 &&
+             (chunks == 3 || (sparse && (chunks % 2 == 1 || p->num_samples >= kRandomSortMinSamples)))))
+            NG = 1;
+    }
     const int C = p->latents.channels, G = p->latents.num_grids;
     // 16-channel grids, or the reference network's four 3-channel grids.
     const bool c3 = plan->shape == kShapeRef;
@@ -665,7 +675,10 @@ void plan16(const nt_params *p, nt_kernel_type type, TrainPlan *plan, int flags)
     // samples (two grids, 2048^2 texels: 231 -> 187 us a step; four, a million of 4096^2: 1,268
     // -> 823), and from 65,536 where there is a sample to at most 32 texels (four grids, 65,536
     // of 512^2: 114 -> 84 us; 131,072 of 2048^2: 228 -> 182; sparser, 65,536 of 4096^2: 219,
-    // 241 sorted; fewer, 32,768 of 1024^2: 71, 82 sorted).
+    // 241 sorted; fewer, 32,768 of 1024^2: 71, 82 sorted). From 262,144 it gains at any density
+    // but the sparsest, where a wave's boxes pass kPathMaxCells and it costs little (one to 256
+    // texels: four grids 262,144 samples 849 -> 795 us, a million 3,360 -> 3,168; two grids a
+    // million 2,810 -> 2,720, 262,144 659 unsorted, 672 sorted; one to 1,024: equal).
     plan->sort_off = plan->sort_temp = 0;
     const bool sorted = p->num_samples >= kRandomSortMinSamples ||
                         (p->num_samples >= kRandomSortMinDense && 32 * (int64_t)p->num_samples >= texels &&

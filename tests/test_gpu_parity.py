@@ -513,11 +513,11 @@ def test_random_texel_path_scatter_weights(lib, shape, size, grid_sizes, loss_we
 
 @pytest.mark.parametrize("shape", ["c2", "c4"])
 @pytest.mark.parametrize("image,n,max_wg", [(64, 127, 0), (64, 129, 1), (64, 640, 2), (64, 1300, 2), (512, 1300, 2),
-                                            (64, 2100, 3)])
+                                            (64, 2100, 3), (512, 1100, 1), (64, 300, 1)])
 def test_train_step_random_tiles(lib, O, shape, image, n, max_wg):
     """NT_SAMPLES_RANDOM tiles of one, two and four chunks in one and two groups (n samples on at
-    most max_wg workgroups; four sparse grids take one group), the last partial: gradients match
-    the oracle's."""
+    most max_wg workgroups; four grids take one group for three chunks a workgroup and, sparse,
+    for any odd number), the last partial: gradients match the oracle's."""
     say(f"case: random tiles {shape} image {image} samples {n} workgroups {max_wg}")
     nt.check(lib.nt_set_test_hooks(max_wg, 0))
     try:
