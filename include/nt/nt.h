@@ -263,9 +263,11 @@ size_t nt_train_workspace_bytes(const nt_params *params, nt_kernel_type type);
 int nt_profile_next_launch(void *start_event, void *stop_event);
 
 /* Test hooks (no reference counterpart; for this library's own tests, not for production
- * runs). Process-wide, taking effect at the next nt_train_step:
+ * runs). Process-wide, taking effect at the next nt_train_step or nt_inference:
  *   max_train_workgroups > 0 caps the 16-channel train kernel's workgroups (0: one per
- *   compute unit), so that small regions give each workgroup several tiles;
+ *   compute unit), so that small regions give each workgroup several tiles, and lays
+ *   nt_inference's strips out for that many compute units and runs no more workgroups, so
+ *   that small images have strips of up to 16 rows and each wave several of them;
  *   flags bit 0 (NT_HOOK_DROP_MARGINS) removes the margin of that kernel's chunk cell box,
  *   which drives its latent scatter's out-of-box path (per-sample global atomics);
  *   flags bit 1 (NT_HOOK_SORT_RANDOM) makes NT_SAMPLES_RANDOM steps sort their samples by

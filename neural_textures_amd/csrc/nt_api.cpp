@@ -91,6 +91,13 @@ int device_cu_count()
     return cached[dev];
 }
 
+// The CUs that train and inference launches are laid out for: a test hook can lower them.
+int workgroup_cap()
+{
+    const int cus = device_cu_count(), hook = g_hook_max_workgroups.load(std::memory_order_relaxed);
+    return hook > 0 ? std::min(cus, hook) : cus;
+}
+
 int mip_dim_h(int size, int mip)
 {
     int d = size >> mip;
@@ -385,9 +392,7 @@ void plan16(const nt_params *p, nt_kernel_type type, TrainPlan *plan, int flags)
     // (a million, 16 texels: 861 -> 840 us, 12: 767 -> 759, 8: 670 two groups, 690 one, 4: 557 and
     // 633; 262,144, 16 texels: 241 -> 238, 12: 209 both, 11: 199 two groups, 208 one).
     // (A test hook can lower the workgroups, so that small steps loop and take two groups.)
-    int cap = device_cu_count();
-    if (const int hook = g_hook_max_workgroups.load(std::memory_order_relaxed); hook > 0)
-        cap = std::min(cap, hook);
+    const int cap = workgroup_cap();
     if (random && NG == 2 && !(flags & kPlanSmall)) {
         const int64_t chunks = ((int64_t)p->num_samples + kChunk * cap - 1) / (kChunk * cap);
         const bool sparse = 12 * (int64_t)p->num_samples <= texels;
@@ -1745,7 +1750,7 @@ static bool infer_desc(const nt_params *p, const FwdDesc &f, InferDesc &d)
     // give every SIMD four.
     d.strips_x = (W + 31) / 32;
     auto strips_of = [&](int rows) { return (int64_t)d.strips_x * ((H + rows - 1) / rows); };
-    const int64_t waves = 4 * (int64_t)device_cu_count(); // one per SIMD
+    const int64_t waves = 4 * (int64_t)workgroup_cap(); // one per SIMD
     d.rows = strips_of(16) >= 8 * waves ? 16 : 8;
     while (d.rows > 1 && strips_of(d.rows) < 4 * waves)
         d.rows /= 2;
@@ -1755,6 +1760,8 @@ static bool infer_desc(const nt_params *p, const FwdDesc &f, InferDesc &d)
     const int64_t strips = (int64_t)d.strips_x * d.strips_y;
     d.blocks = (int)std::min<int64_t>((strips + kFwdWaves - 1) / kFwdWaves,
                                       std::min(kFwdMaxBlocks, forward_blocks(f.count) * kFwdWaves));
+    if (const int hook = g_hook_max_workgroups.load(std::memory_order_relaxed); hook > 0)
+        d.blocks = std::min(d.blocks, hook);
     return true;
 }
 

@@ -720,8 +720,8 @@ def test_inference(lib, O, shape):
 
 
 # (network, image size, textures' channels, texture size as the image's or another): strips of
-# one pixel and of 32, 33 and 31 (whole, one over, one short), row counts around the five-row
-# window, the smallest image the strip kernel takes (4 x 4) and one below it, sizes whose texel
+# one pixel and of 32, 33 and 31 (whole, one over, one short), of one row (images this small;
+# test_inference_strip_rows has taller ones), the smallest image the strip kernel takes (4 x 4) and one below it, sizes whose texel
 # centres are not exact in fp32, output rows of 16, 9, 12 and 3 floats, one to five textures.
 INFERENCE_CASES = [
     ("ref", (4, 4), [3, 3, 3], False), ("ref", (3, 9), [3, 3, 3], False), ("ref", (32, 16), [3, 3, 3], False),
@@ -765,6 +765,70 @@ def test_inference_strips(lib, O, shape, size, tex, other_size):
         sync()
         assert_close(gs.inference_output, st.inference_output, "inference output")
         assert abs(float(to_np(gs.inference_mse_accum)[0]) - want) <= 4e-3 * want
+
+
+@pytest.mark.parametrize("shape,size,tex,cus", [
+    # 4 strips across: strips of 16 rows (8 down, the last of 13), of 8 (5, 5), 4 (6, 2) and 2 (6, 1)
+    ("ref", (100, 125), [4, 4, 4, 4], 1), ("ref", (100, 37), [4, 4, 4, 4], 1), ("ref", (128, 22), [4, 4, 4, 4], 1),
+    ("c2", (97, 11), [3, 3, 3], 1),
+    # one texture a lane, and rows of 9, 12 and 3 floats; two strips of 16 rows across
+    ("c1", (100, 125), [3], 1), ("c2", (100, 125), [3, 3, 3], 1), ("c4", (64, 250), [4, 4, 4], 1),
+    # two workgroups; outputs without a texture (target 0)
+    ("c4", (128, 250), [4, 4, 4], 2), ("ref", (100, 125), [3, 3, 3], 1),
+])
+def test_inference_strip_rows(lib, O, shape, size, tex, cus):
+    """Strips of several rows (the row window's five places, its wrap at the image's top and
+    bottom), several a wave: with the textures holding the outputs themselves each pixel's target
+    is its own output, so the SSE is that of the outputs without a texture, up to the taps'
+    weights (a texel centre's position is within two roundings of size * 2^-24, so a target within
+    2^-13 of the largest output here). Any other row's target is a whole output away: checked with
+    the textures rolled by a row."""
+    import torch
+    w, h = size
+    say(f"case: inference strip rows {shape} {size} textures {tex} compute units {cus}")
+    rng = np.random.default_rng(w * 1000 + h)
+    st = make_state(shape, image=64, region=(16, 16), seed=w)
+    for l in range(st.net.num_layers):
+        st.net.biases[l] = P.f16_bits(rng.uniform(-0.1, 0.1, st.net.sizes[l + 1]))
+    st.image_width, st.image_height = w, h
+    no, used = st.net.sizes[-1], sum(tex)
+    st.textures = [P.make_texture(w, h, c, np.zeros((h, w, 4), np.float32)) for c in tex]
+    st.inference_output = np.zeros(w * h * no, np.float32)
+    st.inference_mse_accum = np.zeros(1, np.float32)
+    assert O.ntref_inference(C.byref(st.params())) == 0
+    gs = st.to_torch()
+    need = lib.nt_inference_workspace_bytes(C.byref(gs.params()))
+
+    def infer(ws):
+        gs.workspace = torch.empty(need, dtype=torch.uint8, device="cuda") if ws else None
+        gs.inference_output.fill_(float("nan"))
+        gs.inference_mse_accum.zero_()
+        nt.check(lib.nt_set_test_hooks(cus, 0))
+        try:
+            nt.check(lib.nt_inference(C.byref(gs.params()), None))
+            sync()
+        finally:
+            nt.check(lib.nt_set_test_hooks(0, 0))
+        return to_np(gs.inference_output).reshape(h, w, no).copy(), float(to_np(gs.inference_mse_accum)[0])
+
+    out, _ = infer(True)
+    assert_close(out.reshape(-1), st.inference_output, "inference output")
+    sse = {}
+    for roll in (0, 1):
+        first = 0
+        for t, c in zip(gs.textures, tex):
+            x = np.zeros((h, w, 4), np.float32)
+            x[:, :, :c] = np.roll(out[:, :, first:first + c], roll, axis=0)
+            t.texels = torch.from_numpy(x.reshape(-1)).cuda()
+            first += c
+        for ws in (True, False):
+            again, sse[roll, ws] = infer(ws)
+            assert np.array_equal(again, out)
+    rest = float(np.sum(out[:, :, used:].astype(np.float64) ** 2))
+    bound = w * h * used * (2.0 ** -13 * float(np.abs(out).max())) ** 2 + 1e-5 * rest
+    for ws in (True, False):
+        assert abs(sse[0, ws] - rest) <= bound
+        assert sse[1, ws] - rest > 100 * bound
 
 
 def test_inference_sse_fixed_order(lib, O):
