@@ -272,16 +272,21 @@ int nt_profile_next_launch(void *start_event, void *stop_event);
  *   which drives its latent scatter's out-of-box path (per-sample global atomics);
  *   flags bit 1 (NT_HOOK_SORT_RANDOM) makes NT_SAMPLES_RANDOM steps sort their samples by
  *   bin at any sample count (they do from 262,144 samples, or 65,536 where there is one to
- *   at most 32 image texels), so that small tests reach the sorted order.
+ *   at most 32 image texels), so that small tests reach the sorted order;
+ *   flags bit 2 (NT_HOOK_PATH_ORDER): nt_random_sample_order includes the path (below).
  * nt_set_test_hooks(0, 0) restores the defaults. */
 #define NT_HOOK_DROP_MARGINS 1
 #define NT_HOOK_SORT_RANDOM 2
+#define NT_HOOK_PATH_ORDER 4
 int nt_set_test_hooks(int max_train_workgroups, int flags);
 /* Test hook (no reference counterpart): the order in which nt_train_step with these
- * parameters (NT_UNCONSTRAINED) would read its NT_SAMPLES_RANDOM samples, written to
+ * parameters (NT_UNCONSTRAINED) sorts its NT_SAMPLES_RANDOM samples, written to
  * order[0 .. num_samples) on the device: the sample indices sorted stably by the
- * 64 x 64-texel bin (row-major over the image) of their texels (the step then walks each
- * tile of 1,024 of them along a path through its bins). Uses params->workspace
+ * 64 x 64-texel bin (row-major over the image) of their texels. The step reads them with each
+ * 1,024 of these entries sorted again, stably, along a path through their bins (the four
+ * 16-texel-wide strips of a bin from left to right, in steps of four rows, downwards in the
+ * first and third, upwards in the others); with NT_HOOK_PATH_ORDER that final order is
+ * written. Uses params->workspace
  * (nt_train_workspace_bytes). NT_ERR_UNSUPPORTED when the step trains in slot order
  * (fewer samples than that without NT_HOOK_SORT_RANDOM, or another kernel). */
 int nt_random_sample_order(const nt_params *params, uint32_t *order, void *stream);

@@ -25,6 +25,7 @@ thread_local char g_error[512] = "";
 std::atomic<int> g_hook_max_workgroups{0};
 std::atomic<int> g_hook_no_margins{0};
 std::atomic<int> g_hook_sort_random{0};
+std::atomic<int> g_hook_path_order{0};
 thread_local hipEvent_t g_prof_start = nullptr;
 thread_local hipEvent_t g_prof_stop = nullptr;
 
@@ -1060,11 +1061,12 @@ int nt_set_test_hooks(int max_train_workgroups, int flags)
 {
     if (max_train_workgroups < 0)
         return fail(NT_ERR_INVALID_ARGUMENT, "max_train_workgroups %d", max_train_workgroups);
-    if (flags & ~(NT_HOOK_DROP_MARGINS | NT_HOOK_SORT_RANDOM))
+    if (flags & ~(NT_HOOK_DROP_MARGINS | NT_HOOK_SORT_RANDOM | NT_HOOK_PATH_ORDER))
         return fail(NT_ERR_INVALID_ARGUMENT, "test hook flags %d", flags);
     g_hook_max_workgroups.store(max_train_workgroups, std::memory_order_relaxed);
     g_hook_no_margins.store(flags & NT_HOOK_DROP_MARGINS ? 1 : 0, std::memory_order_relaxed);
     g_hook_sort_random.store(flags & NT_HOOK_SORT_RANDOM ? 1 : 0, std::memory_order_relaxed);
+    g_hook_path_order.store(flags & NT_HOOK_PATH_ORDER ? 1 : 0, std::memory_order_relaxed);
     return ok();
 }
 
@@ -1439,7 +1441,10 @@ int nt_random_sample_order(const nt_params *p, uint32_t *order, void *stream)
         return fail(NT_ERR_MISALIGNED, "workspace must be 16-byte aligned");
     hipStream_t s = (hipStream_t)stream;
     const uint32_t *sorted = nullptr;
-    hipError_t e = launch_random_order(random_order_desc(p, plan, (uint8_t *)p->workspace), s, &sorted);
+    const RandomOrderDesc r = random_order_desc(p, plan, (uint8_t *)p->workspace);
+    hipError_t e = launch_random_order(r, s, &sorted);
+    if (e == hipSuccess && g_hook_path_order.load(std::memory_order_relaxed))
+        e = launch_random_path(r, s);
     if (e == hipSuccess)
         e = hipMemcpyAsync(order, sorted, (size_t)p->num_samples * sizeof(uint32_t), hipMemcpyDeviceToDevice, s);
     if (e != hipSuccess)

@@ -603,6 +603,39 @@ def test_random_sample_order_wave_parts(lib, O, image, region):
     test_random_sample_order_is_the_stable_bin_sort(lib, O, image, region)
 
 
+@pytest.mark.parametrize("image,n", [(64, 1), (64, 64), (100, 1023), (128, 1024), (168, 1025), (2112, 5000)])
+def test_random_path_order(lib, O, image, n):
+    """The order the train kernel reads, exactly: each 1,024 entries of the bin order sorted by
+    bin, path step (16-texel strip, row of four texels, upwards in odd strips) and place; the
+    last tile partial, and the same on a second run."""
+    import torch
+    say(f"case: random path order image {image} samples {n}")
+    st = make_state("c2", image=image, region=(n, 1), seed=29, step=7)
+    st.sample_mode = abi.NT_SAMPLES_RANDOM
+    got = []
+    for flags in (0, abi.NT_HOOK_PATH_ORDER, abi.NT_HOOK_PATH_ORDER):
+        nt.check(lib.nt_set_test_hooks(0, abi.NT_HOOK_SORT_RANDOM | flags))
+        try:
+            g = gpu_workspace(lib, st.to_torch(), abi.NT_UNCONSTRAINED)
+            order = torch.full((n,), -1, dtype=torch.int32, device="cuda")
+            nt.check(lib.nt_random_sample_order(C.byref(g.params()), C.c_void_p(order.data_ptr()), None))
+            sync()
+        finally:
+            nt.check(lib.nt_set_test_hooks(0, 0))
+        got.append(order.cpu().numpy().astype(np.int64))
+    bins, path, again = got
+    assert np.array_equal(np.sort(bins), np.arange(n))
+    key = np.empty(n, np.int64)
+    for slot, i in enumerate(bins):
+        h1 = O.ntref_fmix32(O.ntref_sample_seed(int(i), 7))
+        x, y = (min(int(np.float32(h & 0xFFFFFF) * np.float32(2.0 ** -24) * np.float32(image)), image - 1)
+                for h in (h1, O.ntref_fmix32(h1)))
+        strip, row = (x >> 4) & 3, (y >> 2) & 15
+        key[slot] = ((((y >> 6) * ((image + 63) // 64) + (x >> 6)) * 4 + strip) * 16 + (15 - row if strip & 1 else row))
+    want = np.concatenate([lo + np.argsort(key[lo:lo + 1024], kind="stable") for lo in range(0, n, 1024)])
+    assert np.array_equal(path, bins[want]) and np.array_equal(again, path)
+
+
 def test_train_step_accumulates(lib, O):
     """Two passes without an optimizer step add up (the zero-gradient contract)."""
     say("case: train accumulate")
