@@ -167,9 +167,11 @@ __global__ __launch_bounds__(256) void codec_encode_kernel(const float *values, 
                 us2 kmn = {0xFFFF, 0xFFFF}, kmx = {0, 0};
 #pragma unroll
                 for (int p = 0; p < 16; p += 2) {
-                    // (a NaN gives the lower bound, as fmin(fmax()) does)
-                    v[p] = __builtin_amdgcn_fmed3f(raw[p], -65504.f, 65504.f);
-                    v[p + 1] = __builtin_amdgcn_fmed3f(raw[p + 1], -65504.f, 65504.f);
+                    // (A NaN gives the lower bound, as fmin(fmax()) does: the median of three of
+                    // which one is NaN is the least of the three, taken from the first on, where
+                    // a signalling NaN turns quiet and the bound that follows last remains.)
+                    v[p] = __builtin_amdgcn_fmed3f(raw[p], 65504.f, -65504.f);
+                    v[p + 1] = __builtin_amdgcn_fmed3f(raw[p + 1], 65504.f, -65504.f);
                     const f2 pv = {v[p], v[p + 1]};
                     const us2 hb = __builtin_bit_cast(us2, __builtin_convertvector(pv, h2));
                     const us2 sg = __builtin_bit_cast(us2, __builtin_bit_cast(s2, hb) >> (short)15);

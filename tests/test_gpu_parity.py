@@ -963,6 +963,32 @@ def test_codec_encode_key_spans(lib, O, span):
     assert np.array_equal(gb.cpu().numpy(), want)
 
 
+@pytest.mark.parametrize("w,h,c", [(64, 8, 16), (37, 22, 8), (20, 12, 12), (9, 13, 4)])
+@pytest.mark.parametrize("scale", [0.5, 1e-6, 3e4])
+def test_codec_encode_special_values(lib, O, w, h, c, scale):
+    """Infinities, values past fp16, subnormals, both zeros and NaNs of either sign among ordinary
+    values, in whole and in partial blocks: the oracle's bytes. A signalling NaN encodes as a quiet
+    one, as the lower bound (the oracle gets it quieted: what C's fmax makes of it is open)."""
+    import torch
+    say(f"case: codec special values {w}x{h}x{c} scale {scale}")
+    rng = np.random.default_rng(w * c)
+    v = (rng.standard_normal(w * h * c) * scale).astype(np.float32)
+    nans = np.array([0x7F800001, 0xFF800001, 0x7FBFFFFF, 0x7FC00000, 0xFFC00000, 0x7FFFFFFF], np.uint32).view(np.float32)
+    special = np.array([np.inf, -np.inf, 0.0, -0.0, 6e-8, -6e-8, 3e-5, 65504, 65520, -65520, 1e30, -1e30], np.float32)
+    at = rng.random(v.size) < 0.05
+    v.view(np.uint32)[at] = rng.choice(np.concatenate([nans, special]).view(np.uint32), int(at.sum()))
+    assert np.any(np.isnan(v)) and np.any(np.isinf(v))
+    quiet = v.copy()
+    quiet.view(np.uint32)[np.isnan(v)] |= 0x00400000
+    want = np.zeros(((w + 3) // 4) * ((h + 3) // 4) * 12 * c, np.uint8)
+    assert O.ntref_codec_encode(quiet.ctypes.data, w, h, c, want.ctypes.data) == 0
+    gv = torch.from_numpy(v.view(np.int32)).cuda()
+    gb = torch.zeros(want.size, dtype=torch.uint8, device="cuda")
+    nt.check(lib.nt_codec_encode(gv.data_ptr(), w, h, c, gb.data_ptr(), None))
+    sync()
+    assert np.array_equal(gb.cpu().numpy(), want)
+
+
 @pytest.mark.parametrize("shape,W,H,jitter,mip_min,mip_max", [
     ("c4", 96, 96, 1.0, 0.0, 3.0),
     ("c4", 100, 37, -1.5, 0.5, 6.0),   # ragged blocks, negative jitter, mips past the last one
