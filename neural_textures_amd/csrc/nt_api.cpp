@@ -562,7 +562,7 @@ void plan16(const nt_params *p, nt_kernel_type type, TrainPlan *plan, int flags)
             wcols += 8;
         d.wcols = wcols;
         // Random texels: the slots, or (bin order) each wave's weight rows of one pass.
-        const size_t slots = std::max((size_t)4 * 32 * G * 4 * 8, 3 * (size_t)kChunk * path_stride(G, NG) * 2);
+        const size_t slots = std::max((size_t)4 * 32 * G * 4 * 8, 3 * (size_t)kChunk * path_stride(G) * 2);
         const size_t scatter = dx_rows + (random ? slots : 2 * (size_t)kChunk * wcols * 2);
         size_t un = train16_transpose_bytes(plan->shape);
         un = scatter > un ? scatter : un;

@@ -1013,18 +1013,18 @@ __device__ __forceinline__ void wave_sync()
 // texels) is 0.69, 0.79, 0.93 and 1.14 times 2^-24 of theirs, with fp32 products added one by
 // one 0.78, 1.12, 2.08 and 4.12. With two halves of w itself, whose low one is subnormal for
 // small weights, it was 0.94, 0.95, 1.04 and 1.18, single texels were 2 % off and the smallest
-// weights lost, for 811 us a step instead of 840.
+// weights lost, for 811 us a step instead of 836.
 // What bounds the random-texel kernel: before, its atomics (all performed past the L2: 1.07 GB
 // of records for four grids and a million samples, 600 us of 1,127); now the scattered taps
-// (245 us) and the MLP (335 us). Four grids, 1,048,576 samples of 4096^2 texels: 105 records a
-// wave instead of 512, WRITE_SIZE 1,184 -> 373 MB, kernel 1,127 -> 709 us; two grids, 262,144
-// samples of 2048^2: 172 -> 116 us.
-template <int DS, int G, int NG>
+// (245 us) and the MLP (335 us). Four grids, 1,048,576 samples of 4096^2 texels: 1,212 -> 221 MB
+// written a launch, kernel 1,127 -> 687 us; two grids, 262,144 samples of 2048^2: 142 -> 49 MB,
+// 172 -> 120 us.
+template <int DS, int G>
 __device__ __forceinline__ void scatter_path(const Train16Desc &d, const Grid16 (&own)[G / 2], const _Float16 *dxw,
                                              _Float16 *wrow, const h8 (&dx0)[G], float u, float v, bool valid, int c,
                                              int g, int lane)
 {
-    constexpr int J = G / 2, kCells = path_cells(G, NG), kStride = path_stride(G, NG);
+    constexpr int J = G / 2, kCells = path_cells(G), kStride = path_stride(G);
     const int i16 = lane & 15, grp = lane >> 4;
     uint32_t top = 0; // the largest |dX0| bits, two halves
 #pragma unroll
@@ -1535,8 +1535,8 @@ __global__ __launch_bounds__(kTrainThreads *NG) void train16_kernel(Train16Desc 
         store_rows<KQ0, dx_stride(S::K0)>(dxs, dx0, col, g);
         if constexpr (RND && ORD) {
             // Bin order: only the wave's own rows are read and written, so no barrier.
-            scatter_path<dx_stride(S::K0), G, NG>(d, own, dxs + 32 * wave * dx_stride(S::K0),
-                                                  whi + wave * (96 * path_stride(G, NG)), dx0, u, v, valid, c, g, lane);
+            scatter_path<dx_stride(S::K0), G>(d, own, dxs + 32 * wave * dx_stride(S::K0),
+                                              whi + wave * (96 * path_stride(G)), dx0, u, v, valid, c, g, lane);
         } else if constexpr (RND) {
             // Random texels: no two samples of a chunk are expected to share a texel, so each
             // sample's corners go straight to the gradients (train.cu:460-509's per-sample
