@@ -52,8 +52,8 @@ TRAIN_HBM_BYTES_PER_LAUNCH = {0: (7102.0 * 2.0 + 4181.4) * 1024,
 # gradient read-modify-write (2 x that) + the targets' channels at 16 taps x 4 B.
 RANDOM_BYTES_PER_SAMPLE = {2: 2 * 4 * 64 * 3 + 16 * 9 * 4,    # 2,112
                            4: 4 * 4 * 64 * 3 + 16 * 12 * 4}   # 3,840
-TRAIN_HBM_BYTES_RANDOM = {2: (136317.8 * 2.0 + 47634.2) * 1024,    # same counters, config 2 random texels
-                          4: (530439.0 * 2.0 + 216123.2) * 1024}   # and config 4 random texels (both bin-sorted)
+TRAIN_HBM_BYTES_RANDOM = {2: (136072.9 * 2.0 + 47634.2) * 1024,    # same counters, config 2 random texels
+                          4: (530535.3 * 2.0 + 216125.5) * 1024}   # and config 4 random texels (both bin-sorted)
 # The BC6 block phase's train kernel (the reference network on texels expanded from its
 # BCf-2k block records), same counters.
 TRAIN_HBM_BYTES_BC6 = (9164.0 * 2.0 + 8478.2) * 1024
