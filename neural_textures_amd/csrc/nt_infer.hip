@@ -254,6 +254,10 @@ __global__ __launch_bounds__(kFwdThreads, 2) void inference_kernel(InferDesc d)
             float wy[4];
             const int gy = __builtin_amdgcn_readfirstlane(cr_axis(v, H, wy));
             const bool late = gy == y - 1;
+            // A lane's targets may fall among the zeros that the pixel's other lane stored.
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 #pragma unroll
             for (int j = 0; j < NT; ++j) {
                 float t4[4];
